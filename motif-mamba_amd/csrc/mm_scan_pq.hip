@@ -28,8 +28,11 @@
 //       * Per-lane partial sums of y = sum_n C_n h_n go back through LDS; the owner of the step adds
 //         the LPR partials in lane order, applies D u and the silu(z) gate and stores.
 //       * Global loads for tile i+1 are issued before the scan of tile i.
+//   scan_fwd_pq_step<T, LPR, U>   one time step, four states per lane (the Motif decode step).
+//   scan_fwd_pq_lanes<T, LPR, R>   four states per lane in registers, any strides and lengths,
+//       constant B/C: whatever else the tiled kernel does not take.
 //   scan_fwd_pq_rowlane<T>   one lane per row, the row's states in LDS, P/Q read through the cache
-//       every step: any dstate <= 256, constant B/C, any strides and lengths.
+//       every step: the same for dstate 65 to 256.
 #include <hip/hip_runtime.h>
 
 #include <stdlib.h>
@@ -473,7 +476,252 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
 }
 
 // ------------------------------------------------------------------------------------------------
-// General kernel: one lane per (batch, channel) row; the row's states in LDS (dstate x 64 floats per
+// scan_fwd_pq_step<T, LPR>: one time step (seqlen 1) with variable B and C, dstate <= 4 LPR: what the
+// Motif module's decode step calls. From the zero state Q h is zero, so the coupling's contribution per
+// state, P (Q 0), is the same for every batch row: formed once per lane, it keeps the general
+// kernels' result for non-finite P, Q and decays. LPR lanes share a (batch, channel) row, four states
+// each, and serve U batch rows with one load of A, P and Q, every row's loads issued before the
+// first is used. The call moves little more than the final states, which leave as 16-byte stores of
+// consecutive lanes (one lane per row wrote each 64-byte state row in 4-byte pieces). 64 x 4,096
+// channels, dstate 16, rank 2, fp16 (20 MB): 47.5 us with one lane per row, 16.8 us here
+// (the kernel alone; 25 us when every lane also loaded its P and Q element by element for one row).
+// ------------------------------------------------------------------------------------------------
+constexpr int kLanesBlock = 256;
+
+template <typename T, int LPR, int U>
+__global__ void __launch_bounds__(kLanesBlock)
+scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t bc_vec) {
+    constexpr int S = 4;
+    const int k = threadIdx.x % LPR;       // states 4 k .. 4 k + 3
+    const int64_t d_raw = int64_t(blockIdx.x) * (kLanesBlock / LPR) + threadIdx.x / LPR;
+    const bool active = d_raw < p.dim;
+    const int64_t d = active ? d_raw : p.dim - 1;  // clamped for loads; stores are predicated
+    const int64_t g = d / ratio;
+    const int N = int(p.dstate);
+    const int n0 = S * k;
+    int nn[S];
+    bool on[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        on[s] = n0 + s < N;
+        nn[s] = on[s] ? n0 + s : N - 1;
+    }
+
+    T uv[U], dv[U], zv[U], bv[U][S], cv[U][S];
+    const int64_t ou = d * p.u_d_stride, od = d * p.delta_d_stride, oz = d * p.z_d_stride;
+    const int64_t b0 = int64_t(blockIdx.y) * U;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
+        uv[i] = (reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride)[ou];
+        dv[i] = (reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride)[od];
+        if (p.z) zv[i] = (reinterpret_cast<const T *>(p.z) + b * p.z_batch_stride)[oz];
+    }
+    struct alignas(S * sizeof(T)) Four {
+        T v[S];
+    };
+    if (bc_vec) {                          // consecutive, aligned states (uniform); no padded state in a lane
+        const int64_t ob = g * p.B_group_stride + (n0 < N ? n0 : 0), oc = g * p.C_group_stride + (n0 < N ? n0 : 0);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
+            const Four fb = *reinterpret_cast<const Four *>(reinterpret_cast<const T *>(p.B) + b * p.B_batch_stride + ob);
+            const Four fc = *reinterpret_cast<const Four *>(reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride + oc);
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                bv[i][s] = fb.v[s];
+                cv[i][s] = fc.v[s];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int64_t ob = g * p.B_group_stride + nn[s] * p.B_dstate_stride;
+            const int64_t oc = g * p.C_group_stride + nn[s] * p.C_dstate_stride;
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
+                bv[i][s] = (reinterpret_cast<const T *>(p.B) + b * p.B_batch_stride)[ob];
+                cv[i][s] = (reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride)[oc];
+            }
+        }
+    }
+    float A2[S], coup[S] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < S; ++s) A2[s] = on[s] ? p.A[d * p.A_d_stride + nn[s] * p.A_dstate_stride] * kLog2e : 0.f;
+    for (int r = 0; r < int(p.pq_rank); ++r) {
+        float q = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            q = __builtin_fmaf(on[s] ? p.Q[d * p.Q_d_stride + r * p.Q_r_stride + nn[s] * p.Q_dstate_stride] : 0.f, 0.f, q);
+        q = group_sum<LPR>(q);
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            coup[s] = __builtin_fmaf(on[s] ? p.P[d * p.P_d_stride + nn[s] * p.P_dstate_stride + r * p.P_r_stride] : 0.f, q, coup[s]);
+    }
+    const float Dv = p.D ? p.D[d] : 0.f;
+    const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+    const bool ls_vec = N % S == 0 && reinterpret_cast<uintptr_t>(p.last_state) % 16 == 0;
+
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const int64_t b = b0 + i;
+        const bool row = active && b < p.batch;
+        float dt = to_f32(dv[i]) + bias;
+        if (p.delta_softplus) dt = softplus_fast(dt);
+        const float uu = to_f32(uv[i]);
+        const float du = dt * uu;
+        float h[S], y = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float w = __builtin_fmaf(dt, coup[s], du * (on[s] ? to_f32(bv[i][s]) : 0.f));
+            h[s] = __builtin_fmaf(decay_exp2(dt, A2[s]), 0.f, w);
+            y = __builtin_fmaf(h[s], on[s] ? to_f32(cv[i][s]) : 0.f, y);
+        }
+        y = group_sum<LPR>(y);
+        if (row && k == 0) {
+            const float o = p.D ? __builtin_fmaf(Dv, uu, y) : y;
+            if (p.out) (reinterpret_cast<T *>(p.out) + b * p.out_batch_stride)[d * p.out_d_stride] = from_f32<T>(o);
+            if (p.out_z)
+                (reinterpret_cast<T *>(p.out_z) + b * p.out_z_batch_stride)[d * p.out_z_d_stride] = from_f32<T>(o * silu_fast(to_f32(zv[i])));
+        }
+        if (row && p.last_state) {
+            float *ls = p.last_state + (b * p.dim + d) * N + n0;
+            if (ls_vec) {
+                if (n0 < N) *reinterpret_cast<float4 *>(ls) = make_float4(h[0], h[1], h[2], h[3]);
+            } else {
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    if (on[s]) ls[s] = h[s];
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// scan_fwd_pq_lanes<T, LPR, R>: any request with dstate <= 4 LPR -- constant B/C, any strides,
+// alignment and length, every output: what neither the tiled nor the one-step kernel takes. LPR lanes
+// share a (batch, channel) row, four states each in registers with their A, P and Q, the coupling's R
+// sums as DPP butterflies, the next step's inputs in flight during a step.
+// ------------------------------------------------------------------------------------------------
+template <typename T, int LPR, int R>
+__global__ void __launch_bounds__(kLanesBlock)
+scan_fwd_pq_lanes(const mm_scan_fwd_params p, const int64_t ratio) {
+    constexpr int S = 4;
+    const int k = threadIdx.x % LPR;       // states 4 k .. 4 k + 3
+    const int64_t d_raw = int64_t(blockIdx.x) * (kLanesBlock / LPR) + threadIdx.x / LPR;
+    const int64_t b = blockIdx.y;
+    const bool active = d_raw < p.dim;
+    const int64_t d = active ? d_raw : p.dim - 1;  // clamped for loads; stores are predicated
+    const int64_t g = d / ratio;
+    const int64_t L = p.seqlen;
+    const int N = int(p.dstate);
+    const int rank = int(p.pq_rank);
+    const int n0 = S * k;
+
+    float A2[S], Pr[S][R], Qr[R][S], Bc[S], Cc[S];
+    const T *Bv[S], *Cv[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int n = n0 + s;
+        const bool on = n < N;
+        const int nn = on ? n : N - 1;
+        A2[s] = on ? p.A[d * p.A_d_stride + n * p.A_dstate_stride] * kLog2e : 0.f;
+        Bc[s] = on && !p.is_variable_B ? reinterpret_cast<const float *>(p.B)[d * p.B_d_stride + n * p.B_dstate_stride] : 0.f;
+        Cc[s] = on && !p.is_variable_C ? reinterpret_cast<const float *>(p.C)[d * p.C_d_stride + n * p.C_dstate_stride] : 0.f;
+        Bv[s] = reinterpret_cast<const T *>(p.B) + b * p.B_batch_stride + g * p.B_group_stride + nn * p.B_dstate_stride;
+        Cv[s] = reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride + g * p.C_group_stride + nn * p.C_dstate_stride;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool use = on && r < rank;
+            Pr[s][r] = use ? p.P[d * p.P_d_stride + n * p.P_dstate_stride + r * p.P_r_stride] : 0.f;
+            Qr[r][s] = use ? p.Q[d * p.Q_d_stride + r * p.Q_r_stride + n * p.Q_dstate_stride] : 0.f;
+        }
+    }
+    const float Dv = p.D ? p.D[d] : 0.f;
+    const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+    const int64_t n_chunks = (L + MM_SCAN_CHUNK - 1) / MM_SCAN_CHUNK;
+    const T *up = reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride + d * p.u_d_stride;
+    const T *dp = reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride + d * p.delta_d_stride;
+    const T *zp = p.z ? reinterpret_cast<const T *>(p.z) + b * p.z_batch_stride + d * p.z_d_stride : nullptr;
+    T *op = p.out ? reinterpret_cast<T *>(p.out) + b * p.out_batch_stride + d * p.out_d_stride : nullptr;
+    T *ozp = p.out_z ? reinterpret_cast<T *>(p.out_z) + b * p.out_z_batch_stride + d * p.out_z_d_stride : nullptr;
+    struct Step {
+        T u, d, z, b[S], c[S];
+    };
+    auto load = [&](int64_t t) {
+        Step x;
+        x.u = up[t];
+        x.d = dp[t];
+        if (zp) x.z = zp[t];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            if (p.is_variable_B) x.b[s] = Bv[s][t];
+            if (p.is_variable_C) x.c[s] = Cv[s][t];
+        }
+        return x;
+    };
+    float h[S] = {0.f, 0.f, 0.f, 0.f};
+    Step nxt = load(0);
+    for (int64_t t = 0; t < L; ++t) {
+        const Step x = nxt;
+        nxt = load(t + 1 < L ? t + 1 : t);     // in flight during this step
+        if (p.tile_states && active && t % 16 == 0) {
+            // The state before this 16-step tile, for the backward (states past dstate are 0).
+            float *ck = p.tile_states + ((t / 16) * p.batch * p.dim + b * p.dim + d) * 16 + n0;
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                if (n0 + s < 16) ck[s] = h[s];
+        }
+        float dt = to_f32(x.d) + bias;
+        if (p.delta_softplus) dt = softplus_fast(dt);
+        const float uu = to_f32(x.u);
+        const float du = dt * uu;
+        float q[R];                            // dt' (Q h_{t-1})
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float acc = Qr[r][0] * h[0];
+#pragma unroll
+            for (int s = 1; s < S; ++s) acc = __builtin_fmaf(Qr[r][s], h[s], acc);
+            q[r] = group_sum<LPR>(acc) * dt;
+        }
+        float y = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const bool on = n0 + s < N;
+            float w = du * (p.is_variable_B ? (on ? to_f32(x.b[s]) : 0.f) : Bc[s]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) w = __builtin_fmaf(Pr[s][r], q[r], w);
+            h[s] = __builtin_fmaf(decay_exp2(dt, A2[s]), h[s], w);
+            y = __builtin_fmaf(h[s], p.is_variable_C ? (on ? to_f32(x.c[s]) : 0.f) : Cc[s], y);
+        }
+        y = group_sum<LPR>(y);
+        if (active && k == 0) {
+            const float o = p.D ? __builtin_fmaf(Dv, uu, y) : y;
+            if (op) op[t] = from_f32<T>(o);
+            if (ozp) ozp[t] = from_f32<T>(o * silu_fast(to_f32(x.z)));
+        }
+        if (active && p.chunk_states && ((t + 1) % MM_SCAN_CHUNK == 0 || t == L - 1)) {
+            float *cs = p.chunk_states + ((b * p.dim + d) * n_chunks + t / MM_SCAN_CHUNK) * 2 * N;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                if (n0 + s < N) {
+                    cs[2 * (n0 + s)] = 1.f;
+                    cs[2 * (n0 + s) + 1] = h[s];
+                }
+            }
+        }
+    }
+    if (active && p.last_state) {
+        float *ls = p.last_state + (b * p.dim + d) * N + n0;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (n0 + s < N) ls[s] = h[s];
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// dstate past 64: one lane per (batch, channel) row; the row's states in LDS (dstate x 64 floats per
 // block, lane-minor so every access is conflict-free), P and Q read through the cache.
 // ------------------------------------------------------------------------------------------------
 constexpr int kRowBlock = 64;
@@ -630,8 +878,37 @@ int launch_tiled_s(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
     return launch_tiled_sr<T, S, LPR, 8>(p, s);
 }
 
+// One-step requests with variable B and C that write no chunk or tile states take the step kernel:
+// four batch rows per workgroup where that leaves at least one workgroup per SIMD, else one.
+template <typename T, int LPR>
+int launch_lanes(const mm_scan_fwd_params &p, hipStream_t s) {
+    const int64_t dblk = (p.dim + kLanesBlock / LPR - 1) / (kLanesBlock / LPR), ratio = p.dim / p.n_groups;
+    const dim3 grid(unsigned(dblk), unsigned(p.batch)), block(kLanesBlock);
+    if (p.seqlen == 1 && p.is_variable_B && p.is_variable_C && !p.chunk_states && !p.tile_states) {
+        auto vec = [&](const void *ptr, int64_t bs, int64_t gs, int64_t ns) {
+            return reinterpret_cast<uintptr_t>(ptr) % (4 * sizeof(T)) == 0 && bs % 4 == 0 && gs % 4 == 0 && ns == 1;
+        };
+        const int32_t bc_vec = p.dstate % 4 == 0 && vec(p.B, p.B_batch_stride, p.B_group_stride, p.B_dstate_stride) &&
+                               vec(p.C, p.C_batch_stride, p.C_group_stride, p.C_dstate_stride);
+        if (dblk * ((p.batch + 3) / 4) >= device_simds())
+            hipLaunchKernelGGL((scan_fwd_pq_step<T, LPR, 4>), dim3(unsigned(dblk), unsigned((p.batch + 3) / 4)), block,
+                               0, s, p, ratio, bc_vec);
+        else
+            hipLaunchKernelGGL((scan_fwd_pq_step<T, LPR, 1>), grid, block, 0, s, p, ratio, bc_vec);
+        return launch_status("scan_fwd_pq_step");
+    }
+    if (p.pq_rank <= 2) hipLaunchKernelGGL((scan_fwd_pq_lanes<T, LPR, 2>), grid, block, 0, s, p, ratio);
+    else hipLaunchKernelGGL((scan_fwd_pq_lanes<T, LPR, 8>), grid, block, 0, s, p, ratio);
+    return launch_status("scan_fwd_pq_lanes");
+}
+
 template <typename T>
 int launch_rowlane(const mm_scan_fwd_params &p, hipStream_t s) {
+    if (p.seqlen > 0) {
+        if (p.dstate <= 16) return launch_lanes<T, 4>(p, s);
+        if (p.dstate <= 32) return launch_lanes<T, 8>(p, s);
+        if (p.dstate <= 64) return launch_lanes<T, 16>(p, s);
+    }
     dim3 grid(unsigned((p.dim + kRowBlock - 1) / kRowBlock), unsigned(p.batch));
     const size_t lds = size_t(p.dstate) * kRowBlock * sizeof(float);  // <= 64 KB at dstate 256
     hipLaunchKernelGGL((scan_fwd_pq_rowlane<T>), grid, dim3(kRowBlock), lds, s, p, p.dim / p.n_groups);

@@ -386,3 +386,15 @@ def test_pq_argument_errors():
     a = selective_scan_fn(**case)
     b = selective_scan_fn(**case, gamma=torch.randn(8, 16, device=DEV))
     torch.testing.assert_close(a, b, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("N,R,L,batch,dim,bkind", [
+    (16, 2, 1, 18, 16384, "3d"), (5, 1, 1, 3, 70, "3d"), (16, 8, 3, 5, 33, "3d"), (20, 2, 7, 2, 48, "3d"),
+    (32, 2, 33, 2, 40, "const"), (64, 8, 5, 2, 17, "const"), (63, 3, 40, 1, 24, "const")])
+def test_pq_lanes_kernel_edges(N, R, L, batch, dim, bkind):
+    """The one-step kernel (one and several batch rows per workgroup with a remainder) and the lanes
+    kernel (few steps, constant B/C): a partial last channel block, dstate off the 4-state lanes and
+    off the lane count, up to the widest; float32, so the oracle's own tolerance holds."""
+    _say(f"pq lanes N={N} R={R} L={L} batch={batch} dim={dim} {bkind}")
+    case = _pq_case(900 + N + L, batch=batch, dim=dim, L=L, N=N, R=R, dtype=torch.float32, bkind=bkind)
+    _vs_oracle(case, torch.float32, "lanes")
