@@ -41,14 +41,13 @@ int64_t device_simds();
 template <typename T>
 int launch_pq(const mm_scan_fwd_params &p, hipStream_t stream, bool diag_x = false);
 
-// The diagonal scan on the P/Q kernels with a zero rank-1 coupling (mm_scan_pq.hip), for diagonal
-// requests the dstate-16 kernels do not take: diag_via_pq_fwd / diag_via_pq_bwd tell whether a
-// request goes that way (inference forwards with dstate != 16 up to 64; backwards with dstate < 16),
-// attach_zero_pair fills a copy of its parameters with the zero pair (and the gradient sink).
+// The diagonal scan on the P/Q kernels (mm_scan_pq.hip), for requests the dstate-16 kernels do not
+// take: diag_via_pq_fwd tells whether a forward goes that way (dstate != 16 up to 64) with the zero
+// rank-1 pair that attach_zero_pair puts in a copy of its parameters, diag_lanes_bwd whether a
+// backward (dstate <= 64) runs scan_bwd_lanes without a coupling.
 bool diag_via_pq_fwd(const mm_scan_fwd_params &p);
 int attach_zero_pair(mm_scan_fwd_params &q);
-bool diag_via_pq_bwd(const mm_scan_bwd_params &p);
-int attach_zero_pair(mm_scan_bwd_params &q);
+bool diag_lanes_bwd(const mm_scan_bwd_params &p);
 
 // Backward (mm_scan_bwd.hip): clears the accumulated gradients and launches the backward kernels
 // on `stream`; bwd_workspace_bytes() is the scratch it uses best, bwd_workspace_min_bytes() the
@@ -57,14 +56,21 @@ template <typename T>
 int launch_bwd(const mm_scan_bwd_params &p, hipStream_t stream);
 int64_t bwd_workspace_bytes(const mm_scan_bwd_params &p);
 int64_t bwd_workspace_min_bytes(const mm_scan_bwd_params &p);
+// Whether the dstate-16 diagonal backward takes the request, whole or split into groups of 16 states.
+bool bwd_tiled_ok(const mm_scan_bwd_params &p);
 
-// Backward with the low-rank P/Q coupling (mm_scan_pq_bwd.hip): pq_bwd_ok() tells whether the
-// request fits the kernel; launch_pq_bwd() runs it with the checkpoint scratch `ck` and the dB / dC
-// partial slabs (the caller clears the accumulated gradients first and reduces the slabs after).
-bool pq_bwd_ok(const mm_scan_bwd_params &p);
+// Backward with the low-rank P/Q coupling, dstate <= 64 (mm_scan_bwd_lanes.hip): bwd_lanes_ok() tells
+// whether the request fits the kernel; launch_bwd_lanes() runs it on the batch rows of `p` with the
+// checkpoints `ck` ([tile][ck_batch][dim][bwd_lanes_np()]) and the dB / dC partial slabs
+// ([dim / 16 / n_groups][batch][group][bwd_lanes_np()][L up to a multiple of 4]); the caller clears
+// the accumulated gradients first, launches bwd_lanes_batch() rows at a time and reduces the slabs.
+bool bwd_lanes_ok(const mm_scan_bwd_params &p);
+int bwd_lanes_np(const mm_scan_bwd_params &p);
+int64_t bwd_lanes_batch(const mm_scan_bwd_params &p);
 template <typename T>
-int launch_pq_bwd(const mm_scan_bwd_params &p, hipStream_t stream, float *ck, float *partB, float *partC);
-// The P/Q backward for the other shapes (dstate up to 256, constant B or C, any length and channel
+int launch_bwd_lanes(const mm_scan_bwd_params &p, hipStream_t stream, float *ck, int64_t ck_batch, float *partB,
+                     float *partC);
+// The P/Q backward for the other shapes (mm_scan_pq_bwd.hip; dstate up to 256, constant B or C, any length and channel
 // count): one lane per state, checkpoints `ck` of pq_general_ck_floats() floats, float32 atomics.
 template <typename T>
 int launch_pq_general(const mm_scan_bwd_params &p, hipStream_t stream, float *ck, float *partB, float *partC);

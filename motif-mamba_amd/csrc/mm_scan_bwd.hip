@@ -375,7 +375,8 @@ struct BwdSeg {
     int64_t carry_blocks, red_rows, n_blocks;
 };
 
-// dB or dC rows [row0, row1) (row = (b * n_groups + g) * 16 + n), by workgroup wg of n_wg, each of
+// dB or dC rows [row0, row1) (row = (b * n_groups + g) * 2^np_log2 + n, 16 rows per pair in the
+// dstate-16 kernel's slabs), by workgroup wg of n_wg, each of
 // NTH lanes: an element is four steps of a row, the sum of its n_blocks channel-block partials. The
 // blocks are split into K contiguous ranges summed by separate lanes (with K > 1 a short row range
 // still keeps enough loads in flight), each range in block order, and the range sums added in range
@@ -387,18 +388,20 @@ __host__ __device__ __forceinline__ int64_t slab_row(int64_t L) { return (L + 3)
 template <int NTH, int K>
 __device__ __forceinline__ void reduce_slab_rows(const mm_scan_bwd_params &p, const float *part, float *dst,
                                                  int64_t bs, int64_t gs, int64_t ns, int64_t n_blocks, int64_t row0,
-                                                 int64_t row1, int64_t wg, int64_t n_wg, float4 *scratch) {
+                                                 int64_t row1, int64_t wg, int64_t n_wg, float4 *scratch,
+                                                 int np_log2 = 4) {
     constexpr int E = NTH / K;   // elements per workgroup pass
     const int tid = threadIdx.x, e = tid % E, k = tid / E;
     const int64_t Lp = slab_row(p.seqlen), L4 = Lp / 4;
-    const int64_t st = p.batch * p.n_groups * 16 * L4;   // one block's slab, in float4
+    const int64_t st = ((p.batch * p.n_groups) << np_log2) * L4;   // one block's slab, in float4
+    const int64_t np_mask = (int64_t(1) << np_log2) - 1;
     const int64_t b_lo = n_blocks * k / K, b_hi = n_blocks * (k + 1) / K;
     const int64_t end = row1 * L4;
     for (int64_t base = row0 * L4 + wg * E; base < end; base += n_wg * E) {   // uniform over the workgroup
         const int64_t i = base + e;
         const int64_t row = i / L4, t4 = i - row * L4;
-        // Slab rows past dstate (P/Q with dstate < 16) are not written.
-        const bool live = i < end && row % 16 < p.dstate;
+        // Slab rows past dstate (P/Q with dstate < 2^np_log2) are not written.
+        const bool live = i < end && (row & np_mask) < p.dstate;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
         if (live) {
             const float4 *src = reinterpret_cast<const float4 *>(part + row * Lp) + t4;
@@ -427,7 +430,7 @@ __device__ __forceinline__ void reduce_slab_rows(const mm_scan_bwd_params &p, co
                 const float4 v = scratch[kk * E + e];
                 acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
             }
-            const int64_t n = row % 16, bg = row / 16;
+            const int64_t n = row & np_mask, bg = row >> np_log2;
             const int64_t gg = bg % p.n_groups, bb = bg / p.n_groups;
             float *o = dst + bb * bs + gg * gs + n * ns + 4 * t4;
             const float a4[4] = {acc.x, acc.y, acc.z, acc.w};
@@ -842,12 +845,12 @@ scan_bwd_tiled16(const mm_scan_bwd_params p, const int64_t ratio, const FastWs w
 // dB and dC rows [row0, rows) = the sums of the channel blocks' partials, in a fixed order.
 __global__ void __launch_bounds__(256)
 scan_bwd_reduce_bc(const mm_scan_bwd_params p, const float *partB, const float *partC, int64_t n_blocks,
-                   int64_t row0, int64_t rows) {
+                   int64_t row0, int64_t rows, int np_log2) {
     __shared__ float4 scratch[256];
     reduce_slab_rows<256, kRedChunks>(p, partB, p.dB, p.dB_batch_stride, p.dB_group_stride, p.dB_dstate_stride,
-                                      n_blocks, row0, rows, blockIdx.x, gridDim.x, scratch);
+                                      n_blocks, row0, rows, blockIdx.x, gridDim.x, scratch, np_log2);
     reduce_slab_rows<256, kRedChunks>(p, partC, p.dC, p.dC_batch_stride, p.dC_group_stride, p.dC_dstate_stride,
-                                      n_blocks, row0, rows, blockIdx.x, gridDim.x, scratch);
+                                      n_blocks, row0, rows, blockIdx.x, gridDim.x, scratch, np_log2);
 }
 
 // dB / dC from the general kernels' slabs [block][batch][group][dstate][seqlen]: each element the
@@ -1092,12 +1095,13 @@ bool states_pass_ok(const mm_scan_bwd_params &p) {
 // dB and dC rows [row0, row1): the n_blocks channel-block partials of each element summed in a
 // fixed order, one launch.
 int launch_reduce(const mm_scan_bwd_params &p, hipStream_t s, const float *partB, const float *partC,
-                  int64_t n_blocks, int64_t row0, int64_t row1) {
+                  int64_t n_blocks, int64_t row0, int64_t row1, int np_log2 = 4) {
     const int64_t total = (row1 - row0) * (slab_row(p.seqlen) / 4);
     if (total <= 0) return MM_OK;
     constexpr int64_t per_wg = 256 / kRedChunks;   // elements per workgroup pass
     const unsigned blocks = unsigned(std::min<int64_t>((total + per_wg - 1) / per_wg, 8192));
-    hipLaunchKernelGGL(scan_bwd_reduce_bc, dim3(blocks), dim3(256), 0, s, p, partB, partC, n_blocks, row0, row1);
+    hipLaunchKernelGGL(scan_bwd_reduce_bc, dim3(blocks), dim3(256), 0, s, p, partB, partC, n_blocks, row0, row1,
+                       np_log2);
     return launch_status("scan_bwd_reduce_bc");
 }
 
@@ -1218,11 +1222,47 @@ int launch_split(const mm_scan_bwd_params &p, hipStream_t s) {
     return MM_OK;
 }
 
-// The P/Q backward (mm_scan_pq_bwd.hip) with the dB / dC block partials reduced in block order.
+// Workspace of the P/Q backward (mm_scan_bwd_lanes.hip): the checkpoints, unless the forward's tile
+// states serve (they hold 16 states per row), then the slabs of one launch's batch rows.
+bool lanes_own_ck(const mm_scan_bwd_params &p) { return !p.tile_states || p.dstate > 16; }
+int64_t lanes_ck_floats(const mm_scan_bwd_params &p) {
+    return lanes_own_ck(p) ? ((p.seqlen + kFT - 1) / kFT) * p.batch * p.dim * bwd_lanes_np(p) : 0;
+}
+int64_t lanes_part_floats(const mm_scan_bwd_params &p) {
+    return (p.dim / 16) * bwd_lanes_batch(p) * bwd_lanes_np(p) * slab_row(p.seqlen);
+}
+
+// Batch rows [b0, b0 + n) of a backward request.
+mm_scan_bwd_params batch_rows(const mm_scan_bwd_params &p, int64_t b0, int64_t n) {
+    mm_scan_bwd_params q = p;
+    const int64_t eb = p.itype == MM_FLOAT32 ? 4 : 2;
+    auto in = [&](const void *t, int64_t bs) -> const void * { return t ? static_cast<const char *>(t) + b0 * bs * eb : t; };
+    auto out = [&](void *t, int64_t bs) -> void * { return t ? static_cast<char *>(t) + b0 * bs * eb : t; };
+    q.batch = n;
+    q.u = in(p.u, p.u_batch_stride);
+    q.delta = in(p.delta, p.delta_batch_stride);
+    q.z = in(p.z, p.z_batch_stride);
+    q.out = in(p.out, p.out_batch_stride);
+    q.dout = in(p.dout, p.dout_batch_stride);
+    q.B = in(p.B, p.B_batch_stride);
+    q.C = in(p.C, p.C_batch_stride);
+    q.du = out(p.du, p.du_batch_stride);
+    q.ddelta = out(p.ddelta, p.ddelta_batch_stride);
+    q.dz = out(p.dz, p.dz_batch_stride);
+    q.out_z = out(p.out_z, p.out_z_batch_stride);
+    q.dB = p.dB + b0 * p.dB_batch_stride;
+    q.dC = p.dC + b0 * p.dC_batch_stride;
+    return q;
+}
+
+// The P/Q backward (and the diagonal one of other dstate values and lengths): the kernel of mm_scan_bwd_lanes.hip with the dB / dC block partials reduced in
+// block order, a workspace's worth of batch rows at a time, or the general one.
 template <typename T>
-int launch_pq(const mm_scan_bwd_params &p, hipStream_t s) {
-    if (!pq_bwd_ok(p)) {   // the general P/Q backward: checkpoints, then the dB / dC slabs if any
-        float *const ck = static_cast<float *>(p.workspace);
+int launch_pq(const mm_scan_bwd_params &p_in, hipStream_t s) {
+    mm_scan_bwd_params p = p_in;
+    float *const ws = static_cast<float *>(p.workspace);
+    if (!bwd_lanes_ok(p)) {   // the general P/Q backward: checkpoints, then the dB / dC slabs if any
+        float *const ck = ws;
         const int64_t rpb = pq_general_rows_per_block(p), slab = gen_slab_floats(p, rpb);
         float *const partB = slab && p.is_variable_B ? ck + pq_general_ck_floats(p) : nullptr;
         float *const partC = slab && p.is_variable_C ? ck + pq_general_ck_floats(p) + slab : nullptr;
@@ -1230,15 +1270,20 @@ int launch_pq(const mm_scan_bwd_params &p, hipStream_t s) {
         if (rc != MM_OK || !slab) return rc;
         return launch_gen_slab_reduce(p, s, partB, partC, rpb);
     }
-    // Checkpoints: the forward's tile_states when given, else the head of the workspace.
-    float *ws = static_cast<float *>(p.workspace);
-    float *ck = p.tile_states ? const_cast<float *>(p.tile_states) : ws;
-    float *partB = p.tile_states ? ws : ws + fast_ck_floats(p), *partC = partB + fast_part_floats(p);
-    const int rc = launch_pq_bwd<T>(p, s, ck, partB, partC);
-    if (rc != MM_OK) return rc;
-    // Slab rows past dstate are never written; the reduction reads only rows n < 16 of each slab
-    // and writes rows n < dstate (dB / dC hold dstate rows).
-    return launch_reduce(p, s, partB, partC, p.dim / p.n_groups / 16, 0, p.batch * p.n_groups * 16);
+    const int np = bwd_lanes_np(p), np_log2 = np == 16 ? 4 : np == 32 ? 5 : 6;
+    float *const ck = lanes_own_ck(p) ? ws : const_cast<float *>(p.tile_states);
+    float *const partB = ws + lanes_ck_floats(p), *const partC = partB + lanes_part_floats(p);
+    if (lanes_own_ck(p)) p.tile_states = nullptr;
+    const int64_t nb = bwd_lanes_batch(p);
+    for (int64_t b0 = 0; b0 < p.batch; b0 += nb) {
+        const int64_t n = std::min(nb, p.batch - b0);
+        const mm_scan_bwd_params q = batch_rows(p, b0, n);
+        int rc = launch_bwd_lanes<T>(q, s, ck + b0 * p.dim * np, p.batch, partB, partC);
+        if (rc != MM_OK) return rc;
+        rc = launch_reduce(q, s, partB, partC, p.dim / p.n_groups / 16, 0, n * p.n_groups * np, np_log2);
+        if (rc != MM_OK) return rc;
+    }
+    return MM_OK;
 }
 
 }  // namespace bwd
@@ -1260,14 +1305,16 @@ int launch_gen_slab_reduce(const mm_scan_bwd_params &p, hipStream_t s, const flo
     return launch_status("gen_slab_reduce");
 }
 
+bool bwd_tiled_ok(const mm_scan_bwd_params &p) { return bwd::fast_ok(p) || bwd::split_ok(p); }
+
 int64_t bwd_workspace_bytes(const mm_scan_bwd_params &p) {
     if (bwd::split_ok(p))   // one part's workspace (reused by every part), then the carried sums
         return ((bwd_workspace_bytes(bwd::split_part(p, 0)) + 255) & ~int64_t(255)) +
                bwd::split_acc_floats(p) * int64_t(sizeof(float));
-    if (p.P && !pq_bwd_ok(p))   // the general P/Q backward: its own checkpoints and the slabs
+    if (p.P && !bwd_lanes_ok(p))   // the general P/Q backward: its own checkpoints and the slabs
         return (pq_general_ck_floats(p) + 2 * gen_slab_floats(p, pq_general_rows_per_block(p))) * int64_t(sizeof(float));
-    if (diag_via_pq_bwd(p))   // the P/Q backward with the zero pair (its own checkpoints without tile states)
-        return ((p.tile_states ? 0 : bwd::fast_ck_floats(p)) + 2 * bwd::fast_part_floats(p)) * int64_t(sizeof(float));
+    if (p.P || diag_lanes_bwd(p))   // scan_bwd_lanes
+        return (bwd::lanes_ck_floats(p) + 2 * bwd::lanes_part_floats(p)) * int64_t(sizeof(float));
     if (!p.P && bwd::fast_ok(p) && p.tile_states)
         return (2 * bwd::fast_part_floats(p) + bwd::carry_floats(bwd::seg_plan_for(p))) * int64_t(sizeof(float));
     if (!p.P && bwd::fast_ok(p) && bwd::states_pass_ok(p)) {
@@ -1278,15 +1325,14 @@ int64_t bwd_workspace_bytes(const mm_scan_bwd_params &p) {
         return (bwd::fast_ck_floats(p) + 2 * bwd::fast_part_floats(p) + bwd::carry_floats(bwd::seg_plan_for(q))) *
                int64_t(sizeof(float));
     }
-    if (p.P && p.tile_states) return 2 * bwd::fast_part_floats(p) * int64_t(sizeof(float));
-    if (p.P || bwd::fast_ok(p)) return (bwd::fast_ck_floats(p) + 2 * bwd::fast_part_floats(p)) * int64_t(sizeof(float));
+    if (bwd::fast_ok(p)) return (bwd::fast_ck_floats(p) + 2 * bwd::fast_part_floats(p)) * int64_t(sizeof(float));
     const int64_t n_tiles = (p.seqlen + bwd::kBT - 1) / bwd::kBT;
     return (p.batch * p.dim * n_tiles * p.dstate + 2 * gen_slab_floats(p, bwd::gen_rows_per_block(p))) *
            int64_t(sizeof(float));
 }
 
 int64_t bwd_workspace_min_bytes(const mm_scan_bwd_params &p) {
-    if (diag_via_pq_bwd(p) || bwd::split_ok(p)) return bwd_workspace_bytes(p);
+    if (diag_lanes_bwd(p) || bwd::split_ok(p)) return bwd_workspace_bytes(p);
     if (!p.P && bwd::fast_ok(p) && p.tile_states) return 2 * bwd::fast_part_floats(p) * int64_t(sizeof(float));
     if (!p.P && bwd::fast_ok(p)) return (bwd::fast_ck_floats(p) + 2 * bwd::fast_part_floats(p)) * int64_t(sizeof(float));
     return bwd_workspace_bytes(p);
@@ -1294,12 +1340,11 @@ int64_t bwd_workspace_min_bytes(const mm_scan_bwd_params &p) {
 
 template <typename T>
 int launch_bwd(const mm_scan_bwd_params &p_in, hipStream_t s) {
-    // Diagonal requests with dstate < 16 run the P/Q backward with a zero rank-1 pair.
-    mm_scan_bwd_params p = p_in;
-    if (diag_via_pq_bwd(p_in) && attach_zero_pair(p) != MM_OK) p = p_in;
-    // The accumulated gradients start from zero on the launch stream (the dstate-16 kernel writes
-    // dB and dC whole and only accumulates dA, dD and ddelta_bias).
-    const bool fast = bwd::fast_ok(p) && p.seqlen > 0;
+    const mm_scan_bwd_params &p = p_in;
+    const bool lanes = p.P ? bwd_lanes_ok(p) : diag_lanes_bwd(p);
+    // The accumulated gradients start from zero on the launch stream (the kernels with dB / dC slabs
+    // write those whole and only accumulate the parameters' gradients).
+    const bool fast = p.seqlen > 0 && (lanes || bwd::fast_ok(p));
     bwd::Fills f;
     f.add(p.dA, 1, 1, p.dim, p.dstate, 0, 0, p.dA_d_stride, p.dA_dstate_stride);
     if (p.is_variable_B && !fast)
@@ -1320,7 +1365,7 @@ int launch_bwd(const mm_scan_bwd_params &p_in, hipStream_t s) {
     const int rc = f.launch(s);
     if (rc != MM_OK) return rc;
     if (p.seqlen == 0) return MM_OK;
-    if (p.P) return bwd::launch_pq<T>(p, s);
+    if (p.P || lanes) return bwd::launch_pq<T>(p, s);
     if (bwd::fast_ok(p)) return bwd::launch_fast<T>(p, s);
     if (bwd::split_ok(p)) return bwd::launch_split<T>(p, s);
     return bwd::launch_general<T>(p, s);

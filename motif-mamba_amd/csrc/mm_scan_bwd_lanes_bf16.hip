@@ -1,0 +1,4 @@
+// mm_scan_bwd_lanes_bf16.hip -- the bfloat16 instances of the P/Q backward kernel of
+// mm_scan_bwd_lanes.hip (compiled once per input type, so that the three sets build in parallel).
+#define MM_BWD_LANES_TYPE bf16_t
+#include "mm_scan_bwd_lanes.hip"

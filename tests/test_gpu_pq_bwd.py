@@ -465,3 +465,62 @@ def test_pq_training_step_graph_replay_matches_eager():
         for i, (a, b) in enumerate(zip(got, exp)):
             tol = 1e-5 if i in atomic else 0.0
             torch.testing.assert_close(a, b, rtol=tol, atol=tol, msg=lambda m: f"replay {rep}, output {i}: {m}")
+
+
+@pytest.mark.parametrize("N,R,L,per_dim", [(16, 2, 15, True), (16, 8, 33, True), (1, 1, 1, True), (17, 4, 16, False),
+                                           (32, 8, 31, True), (33, 3, 17, True), (64, 4, 47, False), (63, 2, 32, True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["fp32", "fp16"])
+def test_pq_bwd_lanes_edges(N, R, L, per_dim, dtype, monkeypatch):
+    """The three lane layouts at the edges of their dstate, rank and tile ranges, on rows of any length
+    and alignment (the training padding off; u, z and dout odd-offset views), two groups."""
+    _say(f"pq bwd lanes N={N} R={R} L={L} per_dim={per_dim} {dtype}")
+    monkeypatch.setenv("MM_SCAN_PAD", "0")
+    case = _pq_case(830 + N + L, batch=2, dim=32, L=L, N=N, R=R, dtype=dtype, bkind="4d", G=2, per_dim=per_dim)
+    dout = _dout(831, (2, 32, L), dtype)
+    from motif_mamba_amd import selective_scan_fn
+
+    def off(t):                       # the same values as rows of an (L + 3)-wide tensor, from column 1
+        w = torch.zeros(*t.shape[:-1], L + 3, dtype=t.dtype, device=DEV)
+        w[..., 1:L + 1] = t.to(DEV)
+        return w[..., 1:L + 1]
+
+    g = {k: (v.to(DEV) if torch.is_tensor(v) else v) for k, v in case.items()}
+    g["u"], g["z"] = off(case["u"]), off(case["z"])
+    for n in NAMES:
+        g[n] = g[n].detach().requires_grad_(True)
+    out = selective_scan_fn(**g)
+    grads = torch.autograd.grad(out, [g[n] for n in NAMES], off(dout))
+    torch.cuda.synchronize()
+    exact = selective_scan_pq_bwd_ref(**case, dout=dout)
+    for n, gr in zip(NAMES, grads):
+        _check(gr, exact["d" + n], dtype, f"lanes d{n}")
+
+
+def test_pq_bwd_batch_rows_in_several_launches():
+    """Slabs of five batch rows exceed the 4 GiB one launch takes: four rows, then one. Each row's own
+    gradients equal those of the row alone bit for bit; the parameters' are their sum (float32
+    atomics: a few roundings of the sum's scale)."""
+    _say("pq bwd batch in several launches")
+    from motif_mamba_amd import selective_scan_fn
+    b, d, L, N, R = 5, 4096, 8192, 64, 2
+    gen = torch.Generator(device=DEV).manual_seed(77)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=gen)   # noqa: E731
+    t = dict(u=rn(b, d, L).bfloat16(), delta=(rn(b, d, L) - 4).bfloat16(), A=-(rn(d, N).abs() + 0.5), B=rn(b, N, L).bfloat16(),
+             C=rn(b, N, L).bfloat16(), P=rn(d, N, R) * 0.02, Q=rn(d, R, N) * 0.02)
+    dout = rn(b, d, L).bfloat16()
+
+    def grads(rows):
+        x = {k: (v[rows] if k in ("u", "delta", "B", "C") else v).detach().requires_grad_(True) for k, v in t.items()}
+        out = selective_scan_fn(x["u"], x["delta"], x["A"], x["B"], x["C"], delta_softplus=True, P=x["P"], Q=x["Q"])
+        return dict(zip(x, torch.autograd.grad(out, list(x.values()), dout[rows])))
+
+    whole = grads(slice(0, b))
+    total = {}
+    for i in range(b):
+        one = grads(slice(i, i + 1))
+        for n in ("u", "delta", "B", "C"):
+            assert torch.equal(whole[n][i], one[n][0]), (i, n)
+        for n in ("A", "P", "Q"):
+            total[n] = total.get(n, 0) + one[n].double()
+    for n, v in total.items():
+        assert (whole[n].double() - v).abs().max() <= 1e-5 * v.abs().max(), n
