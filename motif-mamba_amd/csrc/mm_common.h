@@ -307,6 +307,57 @@ __device__ __forceinline__ void buffer_store_vecn(__amdgpu_buffer_rsrc_t r, uint
     }
 }
 
+// ---- accesses that need only the element's alignment --------------------------------------------
+// At a uniform base and a 32-bit byte offset per lane. gfx950 global accesses of several dwords run at
+// any alignment; the copies below compile to them.
+
+// One element as raw bits (16-bit types zero-extended).
+template <typename T>
+__device__ __forceinline__ uint32_t load_elem(const char *base, uint32_t off) {
+    if constexpr (sizeof(T) == 4) return *reinterpret_cast<const uint32_t *>(base + off);
+    else return *reinterpret_cast<const uint16_t *>(base + off);
+}
+template <typename T>
+__device__ __forceinline__ void store_elem(char *base, uint32_t off, float x) {
+    *reinterpret_cast<T *>(base + off) = from_f32<T>(x);
+}
+template <typename T>
+__device__ __forceinline__ float elem_f32(uint32_t w) {
+    if constexpr (std::is_same_v<T, float>) return __uint_as_float(w);
+    else if constexpr (std::is_same_v<T, bf16_t>) return __uint_as_float(w << 16);
+    else return float(__builtin_bit_cast(_Float16, uint16_t(w)));
+}
+// N consecutive elements as one vector.
+template <typename T, int N>
+__device__ __forceinline__ RawVec<T, N> load_any(const char *base, uint32_t off) {
+    struct __attribute__((packed, aligned(alignof(T)))) At {
+        RawVec<T, N> v;
+    };
+    return reinterpret_cast<const At *>(base + off)->v;
+}
+template <typename T, int N>
+__device__ __forceinline__ void store_any(char *base, uint32_t off, const float *x) {
+    struct __attribute__((packed, aligned(alignof(T)))) At {
+        RawVec<T, N> v;
+    };
+    RawVec<T, N> r;
+    if constexpr (std::is_same_v<T, float>) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r.w[i] = __float_as_uint(x[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i)
+            r.w[i] = std::is_same_v<T, bf16_t> ? pack_bf16x2(x[2 * i], x[2 * i + 1]) : pack_f16x2(x[2 * i], x[2 * i + 1]);
+    }
+    reinterpret_cast<At *>(base + off)->v = r;
+}
+// Element i of a vector that starts zeroed, from raw bits.
+template <typename T, int N>
+__device__ __forceinline__ void set_raw(RawVec<T, N> &r, int i, uint32_t bits) {
+    if constexpr (sizeof(T) == 4) r.w[i] = bits;
+    else r.w[i / 2] |= bits << (16 * (i % 2));
+}
+
 // ---- Sums over the LPR consecutive lanes of a group (a channel's lanes) with DPP ----
 
 // x + x[lane permuted by CTRL] as one v_add_f32 with a DPP operand (the compiler inserts the DPP

@@ -71,23 +71,6 @@ constexpr int kT = 16;           // steps per tile
 constexpr int kXS = kT + 1;      // sX row stride (float4)
 constexpr int kRS = kCh + 2;     // sRed row stride (float2)
 
-// One element of T at a uniform base and a 32-bit byte offset, as raw bits (16-bit zero-extended).
-template <typename T>
-__device__ __forceinline__ uint32_t load_elem(const char *base, uint32_t off) {
-    if constexpr (sizeof(T) == 4) return *reinterpret_cast<const uint32_t *>(base + off);
-    else return *reinterpret_cast<const uint16_t *>(base + off);
-}
-template <typename T>
-__device__ __forceinline__ void store_elem(char *base, uint32_t off, float x) {
-    *reinterpret_cast<T *>(base + off) = from_f32<T>(x);
-}
-template <typename T>
-__device__ __forceinline__ float elem_f32(uint32_t w) {
-    if constexpr (std::is_same_v<T, float>) return __uint_as_float(w);
-    else if constexpr (std::is_same_v<T, bf16_t>) return __uint_as_float(w << 16);
-    else return float(__builtin_bit_cast(_Float16, uint16_t(w)));
-}
-
 template <int LPR, int S>
 struct Layout {
     static constexpr int NP = LPR * S;

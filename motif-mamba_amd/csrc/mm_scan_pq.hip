@@ -45,6 +45,12 @@
 #include "mm_common.h"
 #include "mm_internal.h"
 
+// Compiled once per input type (mm_scan_pq_{f16,bf16}.hip include this file).
+#ifndef MM_PQ_TYPE
+#define MM_PQ_TYPE float
+#define MM_PQ_COMMON
+#endif
+
 namespace mm {
 namespace pq {
 
@@ -68,7 +74,11 @@ __device__ __forceinline__ void lds_read_vec(const float *src, float *o) {
 
 // DX: the chunk states in the diagonal scan's form, (prod of the decays since step 0, h), for the
 // diagonal requests run with a zero P/Q pair; otherwise (1, h), the P/Q form.
-template <typename T, int S, int LPR, int R, bool DX = false>
+// VEC: every row starts 16-byte aligned and L is a multiple of 8. Without it (any L, any row
+// alignment) the same vectors move through global accesses that need only the element's alignment,
+// and the last, partial tile moves element by element: 3 x 4,320 channels, L 1,797, dstate 16, rank
+// 2, fp16 0.25 ms against 0.45 ms on copies padded to whole tiles.
+template <typename T, int S, int LPR, int R, bool DX = false, bool VEC = true>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t blocks_per_group) {
     constexpr int NP = S * LPR;            // padded states per channel
@@ -209,8 +219,15 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     const bool padded = N < NP;            // uniform
 
     // Loads at or past the end of a row are redirected into the row's last elements (always in
-    // bounds: L is a multiple of 8); the steps they feed are padding with dt' = 0.
+    // bounds: L is a multiple of 8, or element by element); the steps they feed are padding with
+    // dt' = 0 (and, where a lane's steps may be part padding, u = 0).
     const int64_t lastE = L - E;
+    const char *const ub = reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride + dw * p.u_d_stride);
+    const char *const db = reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride + dw * p.delta_d_stride);
+    const char *const zb = reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.z) + (p.z ? b * p.z_batch_stride + dw * p.z_d_stride : 0));
+    const char *const Bb = reinterpret_cast<const char *>(Bg), *const Cb = reinterpret_cast<const char *>(Cg);
+    char *const ob = reinterpret_cast<char *>(reinterpret_cast<T *>(p.out) + (p.out ? b * p.out_batch_stride + dw * p.out_d_stride : 0));
+    char *const ozb = reinterpret_cast<char *>(reinterpret_cast<T *>(p.out_z) + (p.out_z ? b * p.out_z_batch_stride + dw * p.out_z_d_stride : 0));
     // Loads run D tiles ahead: rings of D entries (elements, B/C) whose registers stay fixed (the
     // tile loop is unrolled by D below; copying an entry whose loads are in flight would wait for
     // them). D = 2 where the second entry fits in registers (S <= 2); at S = 4 it would spill.
@@ -219,6 +236,26 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         RawVec<T, E> u, d, z;
     };
     auto load_elems = [&](int64_t t, Elems &e) {
+        if constexpr (!VEC) {
+            if (t + kT <= L) {             // uniform: a whole tile
+                const int64_t so = t * SZ;
+                const uint32_t eo = uint32_t(es) * SZ;
+                e.u = load_any<T, E>(ub + so, fo_u + eo);
+                e.d = load_any<T, E>(db + so, fo_d + eo);
+                if (zp) e.z = load_any<T, E>(zb + so, fo_z + eo);
+                else e.z = {};
+            } else {
+                e = {};
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const uint32_t eo = uint32_t(t + es + i < L ? t + es + i : L - 1) * SZ;
+                    set_raw<T, E>(e.u, i, load_elem<T>(ub, fo_u + eo));
+                    set_raw<T, E>(e.d, i, load_elem<T>(db, fo_d + eo));
+                    if (zp) set_raw<T, E>(e.z, i, load_elem<T>(zb, fo_z + eo));
+                }
+            }
+            return;
+        }
         uint32_t eo, so;
         if (t + kT <= L) {                 // uniform: a whole tile
             eo = uint32_t(es) * SZ;
@@ -236,7 +273,16 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         RawVec<T, 8> b[NU], c[NU];
     };
     auto load_bc = [&](int64_t t0, BCs &r) {
-        if (t0 + kT <= L) {                // uniform: a whole tile
+        if constexpr (!VEC) {
+            if (t0 + kT <= L) {            // uniform: a whole tile
+                const int64_t so = t0 * SZ;
+#pragma unroll
+                for (int i = 0; i < NU; ++i) {
+                    r.b[i] = load_any<T, 8>(Bb + so, fo_B[i] + uint32_t(8 * u_q[i]) * SZ);
+                    r.c[i] = load_any<T, 8>(Cb + so, fo_C[i] + uint32_t(8 * u_q[i]) * SZ);
+                }
+            }                              // the last, partial tile: stage_bc loads it
+        } else if (t0 + kT <= L) {         // uniform: a whole tile
             const uint32_t so = uint32_t(t0) * SZ;
 #pragma unroll
             for (int i = 0; i < NU; ++i) {
@@ -260,7 +306,32 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         }
     };
     // Tile rows [step][B states | C states] as float32 (zeros for padded states and past L).
-    auto stage_bc = [&](const BCs &r) {
+    auto stage_bc = [&](const BCs &r, int64_t t0) {
+        if constexpr (!VEC) {
+            if (t0 + kT > L) {             // uniform: the partial tile, element by element, one unit at a time
+#pragma unroll 1
+                for (int i = 0; i < NU; ++i) {
+                    const int u = lane + 64 * i, n = u / 4, q = u % 4;
+                    const uint32_t ob = uint32_t((n < N ? n : 0) * p.B_dstate_stride) * SZ;
+                    const uint32_t oc = uint32_t((n < N ? n : 0) * p.C_dstate_stride) * SZ;
+                    uint32_t vb[8], vc[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int64_t st = t0 + 8 * q + e;
+                        const uint32_t o = uint32_t(st < L ? st : L - 1) * SZ;
+                        vb[e] = load_elem<T>(Bb, ob + o);
+                        vc[e] = load_elem<T>(Cb, oc + o);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const bool on = n < N && t0 + 8 * q + e < L;
+                        sBC[(8 * q + e) * BCS + n] = on ? elem_f32<T>(vb[e]) : 0.f;
+                        sBC[(8 * q + e) * BCS + n + NP] = on ? elem_f32<T>(vc[e]) : 0.f;
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
             float vb[8], vc[8];
@@ -278,14 +349,15 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     load_elems(0, e0);
     if (D == 2) load_elems(kT, e1);
     load_bc(0, b0);
-    stage_bc(b0);
+    stage_bc(b0, 0);
     if (D == 2) load_bc(kT, b1);
 
     // Tile t0: its elements in ec, its B/C (already staged) in bc, the next tile's B/C in bn (the
     // same entry as bc when D = 1: loaded at the top of the tile, staged at its end).
     auto tile = [&](const int64_t t0, Elems &ec, BCs &bc, const BCs &bn) __attribute__((always_inline)) {
         const int64_t t1 = t0 + kT;
-        const bool ev = t0 + es < L;       // this lane's E elements exist (L is a multiple of E)
+        // This lane's elements exist: all or none of them where L is a multiple of E.
+        auto ev = [&](int i) { return VEC ? t0 + es < L : t0 + es + i < L; };
         float uu[E], dd[E], zz[E];
         unpack_raw<T, E>(ec.u, uu);
         unpack_raw<T, E>(ec.d, dd);
@@ -300,7 +372,10 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         for (int i = 0; i < E; ++i) {
             const float x = dd[i] + bias;
             dtp[i] = softplus ? softplus_fast(x) : x;
-            if (!ev) dtp[i] = 0.f;         // padded steps of a last, partial tile
+            if (!ev(i)) {                  // padded steps of a last, partial tile
+                dtp[i] = 0.f;
+                if constexpr (!VEC) uu[i] = 0.f;
+            }
             dup[i] = dtp[i] * uu[i];
         }
 #pragma unroll
@@ -412,7 +487,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
 #pragma unroll
         for (int t = 0; t < kT; t += 4)
             *reinterpret_cast<float4 *>(&sY[(cw * LPR + k) * kPad + t]) = make_float4(yp[t], yp[t + 1], yp[t + 2], yp[t + 3]);
-        if (t1 < L) stage_bc(bn);
+        if (t1 < L) stage_bc(bn, t1);
         __syncthreads();
 
         // Epilogue: y of (channel, steps es .. es + E - 1) = the LPR partials, added in lane order.
@@ -429,15 +504,26 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
             y[i] = acc.x;
             y[i + 1] = acc.y;
         }
-        if (active && ev) {
+        if (active && ev(0)) {
             float o[E];
 #pragma unroll
             for (int i = 0; i < E; ++i) o[i] = p.D ? __builtin_fmaf(Dv, uu[i], y[i]) : y[i];
-            if (p.out) buffer_store_vecn<T, E>(rs_o, fo_o, uint32_t(t0) * SZ, o);
+            auto put = [&](auto rs, char *base, uint32_t off) __attribute__((always_inline)) {
+                if constexpr (VEC) {
+                    buffer_store_vecn<T, E>(rs, off, uint32_t(t0) * SZ, o);
+                } else if (t1 <= L) {      // uniform
+                    store_any<T, E>(base + t0 * SZ, off, o);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < E; ++i)
+                        if (ev(i)) store_elem<T>(base + t0 * SZ, off + uint32_t(i) * SZ, o[i]);
+                }
+            };
+            if (p.out) put(rs_o, ob, fo_o);
             if (zp) {
 #pragma unroll
                 for (int i = 0; i < E; ++i) o[i] *= silu_fast(zz[i]);
-                buffer_store_vecn<T, E>(rs_oz, fo_oz, uint32_t(t0) * SZ, o);
+                put(rs_oz, ozb, fo_oz);
             }
         }
         if (active && p.chunk_states) {
@@ -828,12 +914,9 @@ static bool offsets_ok(const mm_scan_fwd_params &p) {
 }
 
 // The (S, LPR) of the tiled kernel for this request, or {0, 0} when the request needs the general
-// kernel: variable B and C, dstate <= 64, seqlen >= 8, rows movable as 16-byte vectors, offsets
-// that fit in 32 bits.
-TiledShape tiled_shape(const mm_scan_fwd_params &p) {
-    if (!p.is_variable_B || !p.is_variable_C || p.dstate > 64 || p.seqlen < 8 || !fwd_vector_ok(&p) ||
-        !offsets_ok(p))
-        return {0, 0};
+// kernel: variable B and C, dstate <= 64, seqlen >= 8, offsets that fit in 32 bits.
+static TiledShape tiled_shape(const mm_scan_fwd_params &p) {
+    if (!p.is_variable_B || !p.is_variable_C || p.dstate > 64 || p.seqlen < 8 || !offsets_ok(p)) return {0, 0};
     const int64_t ratio = p.dim / p.n_groups;
     auto waves = [&](int lpr) { return p.batch * p.n_groups * ((ratio + 64 / lpr - 1) / (64 / lpr)); };
     const char *forced = getenv("MM_PQ_LPR");
@@ -859,23 +942,28 @@ TiledShape tiled_shape(const mm_scan_fwd_params &p) {
     return 2 * waves(8) <= 5 * simds ? cands[1] : cands[0];
 }
 
-template <typename T, int S, int LPR, int R, bool DX = false>
+template <typename T, int S, int LPR, int R, bool DX, bool VEC>
 int launch_tiled_sr(const mm_scan_fwd_params &p, hipStream_t s) {
     constexpr int CPW = 64 / LPR;
     const int64_t ratio = p.dim / p.n_groups;
     const int64_t bpg = (ratio + CPW - 1) / CPW;
     dim3 grid(unsigned(bpg * p.n_groups), unsigned(p.batch));
-    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, DX>), grid, dim3(64), 0, s, p, ratio, int32_t(bpg));
+    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, DX, VEC>), grid, dim3(64), 0, s, p, ratio, int32_t(bpg));
     return launch_status("scan_fwd_pq_tiled");
 }
 
 // diag_x: the zero-pair diagonal route, which has rank 1 and wants the diagonal chunk states.
+template <typename T, int S, int LPR, bool VEC>
+int launch_tiled_v(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
+    if (diag_x) return launch_tiled_sr<T, S, LPR, 2, true, VEC>(p, s);
+    if (p.pq_rank <= 2) return launch_tiled_sr<T, S, LPR, 2, false, VEC>(p, s);
+    if (p.pq_rank <= 4) return launch_tiled_sr<T, S, LPR, 4, false, VEC>(p, s);
+    return launch_tiled_sr<T, S, LPR, 8, false, VEC>(p, s);
+}
 template <typename T, int S, int LPR>
 int launch_tiled_s(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
-    if (diag_x) return launch_tiled_sr<T, S, LPR, 2, true>(p, s);
-    if (p.pq_rank <= 2) return launch_tiled_sr<T, S, LPR, 2>(p, s);
-    if (p.pq_rank <= 4) return launch_tiled_sr<T, S, LPR, 4>(p, s);
-    return launch_tiled_sr<T, S, LPR, 8>(p, s);
+    return fwd_vector_ok(&p) ? launch_tiled_v<T, S, LPR, true>(p, s, diag_x)
+                             : launch_tiled_v<T, S, LPR, false>(p, s, diag_x);
 }
 
 // One-step requests with variable B and C that write no chunk or tile states take the step kernel:
@@ -931,9 +1019,9 @@ int launch_pq(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
     return pq::launch_rowlane<T>(p, s);   // not reached with diag_x (diag_via_pq_fwd requires a tiled shape)
 }
 
-template int launch_pq<float>(const mm_scan_fwd_params &, hipStream_t, bool);
-template int launch_pq<f16_t>(const mm_scan_fwd_params &, hipStream_t, bool);
-template int launch_pq<bf16_t>(const mm_scan_fwd_params &, hipStream_t, bool);
+template int launch_pq<MM_PQ_TYPE>(const mm_scan_fwd_params &, hipStream_t, bool);
+
+#ifdef MM_PQ_COMMON
 
 // ------------------------------------------------------------------------------------------------
 // The diagonal scan through the P/Q kernels. A zero rank-1 pair shared by every channel (P = Q = 0)
@@ -993,5 +1081,7 @@ int attach_zero_pair(mm_scan_fwd_params &q) {
 bool diag_lanes_bwd(const mm_scan_bwd_params &p) {
     return !p.P && diag_pq_enabled() && !bwd_tiled_ok(p) && bwd_lanes_ok(p);
 }
+
+#endif  // MM_PQ_COMMON
 
 }  // namespace mm

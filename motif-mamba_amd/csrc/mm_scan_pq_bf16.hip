@@ -1,0 +1,4 @@
+// mm_scan_pq_bf16.hip -- the bfloat16 instances of the P/Q forward kernels of mm_scan_pq.hip (compiled
+// once per input type, so that the three sets build in parallel).
+#define MM_PQ_TYPE bf16_t
+#include "mm_scan_pq.hip"

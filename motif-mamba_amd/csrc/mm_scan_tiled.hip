@@ -1003,6 +1003,12 @@ int launch_k2i(const mm_scan_fwd_params &p, hipStream_t stream) {
 // MODE 1 and 2: SEG 1 scans segments 0 .. n_seg-2 from a zero state for the states alone (YO false)
 // and writes each segment's end state and sum of delta'; SEG 2 scans every segment from its carried
 // state (and delta' prefix) and writes the outputs, last_state from the last segment.
+//
+// RAG: any length and row alignment (inference). The vectors move through global accesses that need
+// only the element's alignment; the tiles that reach past L move element by element, their steps
+// past L with delta' = u = 0 (the identity) and B = C = 0. 2 x 1,536 channels, L 1,777, bf16, in
+// segments: 94 us against 143 us on copies padded in front to whole pairs (five pad copies and
+// their fills, one copy back); 4 x 5,120 channels, L 4,095: 0.47 against 0.75 ms.
 // ---------------------------------------------------------------------------------------------
 template <typename T>
 struct K2SData {                       // one lane's global data for pair iteration i
@@ -1021,7 +1027,7 @@ struct K2SLds {
 // One 16-channel group of batch row b on 128 lanes (tid 0..127, two waves): the body of scan_fwd_k2s,
 // also run twice per workgroup by scan_fwd_mix. Every lane of the workgroup calls __syncthreads()
 // the same number of times (once per 16-step tile, the same tile count for both groups).
-template <typename T, int PF, bool SOFTPLUS, bool CHUNKS, bool HAS_Z, bool HAS_OUT, bool YO, int SEG>
+template <typename T, int PF, bool SOFTPLUS, bool CHUNKS, bool HAS_Z, bool HAS_OUT, bool YO, int SEG, bool RAG = false>
 __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int64_t ratio, const SegArgs &sg,
                                           const int tid, const int64_t b, const int64_t d0, const int seg,
                                           K2SLds &lds) {
@@ -1041,7 +1047,7 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
     const int swc = swz16(c), swe = swz16(ce);   // LDS block permutations of the two channels
     const int64_t g = d0 / ratio;
     const int64_t L = p.seqlen;
-    const int32_t n_pairs = int32_t(L / (2 * kT1));   // L is a multiple of 32 here
+    const int32_t n_pairs = int32_t((L + (RAG ? 2 * kT1 - 1 : 0)) / (2 * kT1));   // L is a multiple of 32 without RAG
     const int64_t n_chunks = (L + MM_SCAN_CHUNK - 1) / MM_SCAN_CHUNK;
     const int32_t pb = SEG ? int32_t(seg * sg.pairs) : 0;                                 // first pair
     const int32_t pe = SEG ? (pb + int32_t(sg.pairs) < n_pairs ? pb + int32_t(sg.pairs) : n_pairs) : n_pairs;
@@ -1082,18 +1088,60 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
     // never used): every access stays inside the rows.
     auto pair_off = [&](int32_t i) { return uint32_t(i < n_pairs ? i : n_pairs - 1) * uint32_t(2 * kT1 * SZ); };
     auto tile_off = [&](int32_t t) { return uint32_t(t < 2 * n_pairs ? t : 2 * n_pairs - 1) * uint32_t(kT1 * SZ); };
+    // RAG: E steps of a row (byte offset fo of the lane's first one) of tile t, element by element
+    // where the tile reaches past L (then redirected to the row's last element).
+    auto rag_elems = [&](const T *base, uint32_t fo, int32_t t) __attribute__((always_inline)) {
+        const int64_t t0 = int64_t(t) * kT1;
+        const char *const rb = reinterpret_cast<const char *>(base);
+        if (t0 + kT1 <= L) return load_any<T, E>(rb + t0 * SZ, fo);
+        RawVec<T, E> v = {};
+        if (t0 >= L) return v;             // nothing of the tile exists
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int64_t at = t0 + es + k < L ? t0 + es + k : L - 1;
+            set_raw<T, E>(v, k, load_elem<T>(rb, fo + uint32_t(at - es) * SZ));
+        }
+        return v;
+    };
     auto load_tile = [&](int32_t t, RawVec<T, E> &u, RawVec<T, E> &dl, RawVec<T, E> &z) {
+        if constexpr (RAG) {
+            u = rag_elems(ub, fo_u, t);
+            dl = rag_elems(db, fo_d, t);
+            if constexpr (HAS_Z) z = rag_elems(zb, fo_z, t);
+            else z = {};
+            return;
+        }
         const uint32_t sof = tile_off(t);
         u = buffer_load_raw<T, E>(rs_u, fo_u, sof);
         dl = buffer_load_raw<T, E>(rs_d, fo_d, sof);
         if constexpr (HAS_Z) z = buffer_load_raw<T, E>(rs_z, fo_z, sof);
         else z = {};
     };
+    auto rag_bc = [&](const T *base, uint32_t fo, int32_t i) __attribute__((always_inline)) {
+        const int64_t t0 = int64_t(i) * (2 * kT1);
+        const char *const rb = reinterpret_cast<const char *>(base);
+        if (t0 + 2 * kT1 <= L) return load_any<T, 4>(rb + t0 * SZ, fo);
+        RawVec<T, 4> v = {};
+        if (t0 >= L) return v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t at = t0 + sb + k;
+            const uint32_t w = load_elem<T>(rb, fo + uint32_t((at < L ? at : L - 1) - sb) * SZ);
+            set_raw<T, 4>(v, k, at < L ? w : 0u);
+        }
+        return v;
+    };
     auto load_data = [&](int32_t i, K2SData<T> &dst) {
-        const uint32_t sof = pair_off(i);
-        dst.b = buffer_load_raw<T, 4>(rs_b, fo_b, sof);
-        if constexpr (YO) dst.c = buffer_load_raw<T, 4>(rs_c, fo_c, sof);
-        else dst.c = {};
+        if constexpr (RAG) {
+            dst.b = rag_bc(Bb, fo_b, i);
+            if constexpr (YO) dst.c = rag_bc(Cb, fo_c, i);
+            else dst.c = {};
+        } else {
+            const uint32_t sof = pair_off(i);
+            dst.b = buffer_load_raw<T, 4>(rs_b, fo_b, sof);
+            if constexpr (YO) dst.c = buffer_load_raw<T, 4>(rs_c, fo_c, sof);
+            else dst.c = {};
+        }
         load_tile(2 * i + 2, dst.u0, dst.d0, dst.z0);
         load_tile(2 * i + 3, dst.u1, dst.d1, dst.z1);
     };
@@ -1103,7 +1151,7 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
     RawVec<T, E> rz[4];
 
     // Prologue of tile t (slot S = t % 4): delta', delta' u of this lane's two elements -> LDS.
-    auto prologue = [&](auto Slot, const RawVec<T, E> &u, const RawVec<T, E> &dl, const RawVec<T, E> &z) {
+    auto prologue = [&](auto Slot, int32_t t, const RawVec<T, E> &u, const RawVec<T, E> &dl, const RawVec<T, E> &z) {
         constexpr int sl = decltype(Slot)::value & 3;
         float uu[E], dd[E], dtp[E];
         unpack_raw<T, E>(u, uu);
@@ -1112,6 +1160,9 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
         for (int k = 0; k < E; ++k) {
             const float x = dd[k] + bias;
             dtp[k] = SOFTPLUS ? softplus_fast(x) : x;
+            if constexpr (RAG) {
+                if (int64_t(t) * kT1 + es + k >= L) dtp[k] = uu[k] = 0.f;
+            }
         }
         *reinterpret_cast<float2 *>(&DT(Slot)[ce * kT1 + (((es >> 2) ^ swe) << 2) + (es & 3)]) = make_float2(dtp[0], dtp[1]);
         *reinterpret_cast<float2 *>(&DU(Slot)[ce * kT1 + (((es >> 2) ^ swe) << 2) + (es & 3)]) = make_float2(dtp[0] * uu[0], dtp[1] * uu[1]);
@@ -1141,11 +1192,26 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
         unpack_raw<T, E>(rz[sl], zz);
         float o[E] = {__builtin_fmaf(Dv, ru[sl][0], a.x), __builtin_fmaf(Dv, ru[sl][1], a.y)};
         const uint32_t sof = uint32_t(t) * uint32_t(kT1 * SZ);
-        if constexpr (HAS_OUT) buffer_store_vec<T, E>(rs_o, fo_o, sof, o);
+        auto put = [&](auto rs, T *base, uint32_t fo) __attribute__((always_inline)) {
+            if constexpr (!RAG) {
+                buffer_store_vec<T, E>(rs, fo, sof, o);
+                return;
+            }
+            const int64_t t0 = int64_t(t) * kT1;
+            char *const rb = reinterpret_cast<char *>(base) + t0 * SZ;
+            if (t0 + kT1 <= L) {           // uniform
+                store_any<T, E>(rb, fo, o);
+            } else {
+#pragma unroll
+                for (int k = 0; k < E; ++k)
+                    if (t0 + es + k < L) store_elem<T>(rb, fo + uint32_t(k) * SZ, o[k]);
+            }
+        };
+        if constexpr (HAS_OUT) put(rs_o, ob, fo_o);
         if constexpr (HAS_Z) {
 #pragma unroll
             for (int k = 0; k < E; ++k) o[k] *= silu_fast(zz[k]);
-            buffer_store_vec<T, E>(rs_oz, fo_oz, sof, o);
+            put(rs_oz, ozb, fo_oz);
         }
     };
 
@@ -1233,8 +1299,8 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
         load_tile(2 * pb + 1, u1, dl1, z1);
 #pragma unroll
         for (int s = 0; s < PF; ++s) load_data(pb + s, ring[s]);
-        prologue(I0{}, u0, dl0, z0);       // tiles 2 pb and 2 pb + 1, slots 0 and 1
-        prologue(I1{}, u1, dl1, z1);
+        prologue(I0{}, 2 * pb, u0, dl0, z0);       // tiles 2 pb and 2 pb + 1, slots 0 and 1
+        prologue(I1{}, 2 * pb + 1, u1, dl1, z1);
     }
     __syncthreads();
     pre_dt = *reinterpret_cast<const float4 *>(&DT(I0{})[c * kT1 + (swc << 2)]);
@@ -1271,12 +1337,12 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
                 load_data(i + PF, ring[S]);
                 // Interval 2i: scan tile 2i, prepare tile 2i + 2, finish tile 2i - 1.
                 scan_tile(I0{}, t0, DT(T2P{}), DU(T2P{}), YB(I0{}), DT(T2P1{}), DU(T2P1{}));
-                prologue(T2P2{}, nxt.u0, nxt.d0, nxt.z0);
+                prologue(T2P2{}, 2 * i + 2, nxt.u0, nxt.d0, nxt.z0);
                 if constexpr (YO) epilogue(T2P3{}, YB(I1{}), i > pb ? 2 * i - 1 : 2 * pb);
                 __syncthreads();
                 // Interval 2i + 1: scan tile 2i + 1, prepare tile 2i + 3, finish tile 2i.
                 scan_tile(I1{}, t0 + kT1, DT(T2P1{}), DU(T2P1{}), YB(I1{}), DT(T2P2{}), DU(T2P2{}));
-                prologue(T2P3{}, nxt.u1, nxt.d1, nxt.z1);
+                prologue(T2P3{}, 2 * i + 3, nxt.u1, nxt.d1, nxt.z1);
                 if constexpr (YO) epilogue(T2P{}, YB(I0{}), 2 * i);
                 __syncthreads();
             }
@@ -1297,11 +1363,11 @@ __device__ __forceinline__ void k2s_group(const mm_scan_fwd_params &p, const int
     }
 }
 
-template <typename T, int PF, bool SOFTPLUS, bool CHUNKS, bool HAS_Z, bool HAS_OUT, bool YO, int SEG = 0>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 8)))
+template <typename T, int PF, bool SOFTPLUS, bool CHUNKS, bool HAS_Z, bool HAS_OUT, bool YO, int SEG = 0, bool RAG = false>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RAG && sizeof(T) == 4 ? 2 : 3, 8)))
 scan_fwd_k2s(const mm_scan_fwd_params p, const int64_t ratio, const SegArgs sg) {
     __shared__ __align__(16) K2SLds lds;
-    k2s_group<T, PF, SOFTPLUS, CHUNKS, HAS_Z, HAS_OUT, YO, SEG>(p, ratio, sg, threadIdx.x, blockIdx.y,
+    k2s_group<T, PF, SOFTPLUS, CHUNKS, HAS_Z, HAS_OUT, YO, SEG, RAG>(p, ratio, sg, threadIdx.x, blockIdx.y,
                                                                 int64_t(blockIdx.x) * kCh, SEG ? int(blockIdx.z) : 0, lds);
 }
 
@@ -1336,12 +1402,6 @@ __device__ __forceinline__ uint32_t buffer_load_elem(__amdgpu_buffer_rsrc_t r, u
         return __builtin_bit_cast(uint32_t, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
     else
         return uint32_t(__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
-}
-template <typename T>
-__device__ __forceinline__ float elem_f32(uint32_t w) {
-    if constexpr (std::is_same_v<T, float>) return __uint_as_float(w);
-    else if constexpr (std::is_same_v<T, bf16_t>) return __uint_as_float(w << 16);
-    else return float(__builtin_bit_cast(_Float16, uint16_t(w)));
 }
 // One float stored as T (bf16 round-to-nearest-even, as buffer_store_vec converts).
 template <typename T>
@@ -1677,6 +1737,38 @@ K2SKernel k2s_seg_full(bool softplus, bool chunks) {
                                   : scan_fwd_k2s<T, 2, false, false, HAS_Z, HAS_OUT, true, 2>);
 }
 
+// Any length and alignment, inference, one pass or (sg.n_seg > 1) segments.
+template <typename T, bool HAS_Z>
+int launch_k2s_ragged_io(const mm_scan_fwd_params &p, hipStream_t stream, const SegArgs &sg) {
+    const int64_t ratio = p.dim / p.n_groups;
+    const unsigned groups = unsigned(p.dim / kCh), batch = unsigned(p.batch), n_seg = unsigned(sg.n_seg);
+    if (n_seg <= 1) {
+        const K2SKernel kern = p.delta_softplus ? scan_fwd_k2s<T, 2, true, false, HAS_Z, !HAS_Z, true, 0, true>
+                                                : scan_fwd_k2s<T, 2, false, false, HAS_Z, !HAS_Z, true, 0, true>;
+        hipLaunchKernelGGL(kern, dim3(groups, batch), dim3(128), 0, stream, p, ratio, kWholeRows);
+        return launch_status("scan_fwd_k2s_ragged");
+    }
+    const K2SKernel states = p.delta_softplus ? scan_fwd_k2s<T, 2, true, false, false, false, false, 1, true>
+                                              : scan_fwd_k2s<T, 2, false, false, false, false, false, 1, true>;
+    const K2SKernel full = p.delta_softplus ? scan_fwd_k2s<T, 2, true, false, HAS_Z, !HAS_Z, true, 2, true>
+                                            : scan_fwd_k2s<T, 2, false, false, HAS_Z, !HAS_Z, true, 2, true>;
+    hipLaunchKernelGGL(states, dim3(groups, batch, n_seg - 1), dim3(128), 0, stream, p, ratio, sg);
+    int rc = launch_status("scan_fwd_k2s_ragged_states");
+    if (rc != MM_OK) return rc;
+    const int64_t rows = p.batch * p.dim;
+    hipLaunchKernelGGL(seg_carry_kernel, dim3(unsigned((rows * 16 + 255) / 256)), dim3(256), 0, stream, p.A,
+                       p.A_d_stride, p.A_dstate_stride, rows, p.dim, sg);
+    rc = launch_status("seg_carry");
+    if (rc != MM_OK) return rc;
+    hipLaunchKernelGGL(full, dim3(groups, batch, n_seg), dim3(128), 0, stream, p, ratio, sg);
+    return launch_status("scan_fwd_k2s_ragged_seg");
+}
+
+template <typename T>
+int launch_k2s_ragged(const mm_scan_fwd_params &p, hipStream_t stream, const SegArgs &sg) {
+    return p.z ? launch_k2s_ragged_io<T, true>(p, stream, sg) : launch_k2s_ragged_io<T, false>(p, stream, sg);
+}
+
 // Segmented scan on k2s (L a multiple of 32): the states of segments 0 .. n_seg-2 (SEG 1), the
 // carry chain, every segment with its outputs (SEG 2). Requests that write both out and out_z, and
 // fp32 requests with chunk states, return MM_ERR_UNSUPPORTED before launching anything (the
@@ -1782,6 +1874,28 @@ static bool k2s_bytes_ok(const mm_scan_fwd_params &p) {
     return span * size < (int64_t(1) << 32);
 }
 
+// Requests of any length and row alignment that the ragged k2s takes: inference (no chunk or tile
+// states, one output), from kMinRagged steps on.
+constexpr int64_t kMinRagged = 8;
+static bool ragged_ok(const mm_scan_fwd_params &p) {
+    if (p.dstate != 16 || !p.is_variable_B || !p.is_variable_C || p.chunk_states || p.tile_states || (p.z && p.out))
+        return false;
+    if (p.dim % tiled::kCh != 0 || (p.dim / p.n_groups) % tiled::kCh != 0) return false;
+    // Rows start on whole elements.
+    const uintptr_t eb = p.itype == MM_FLOAT32 ? 4 : 2;
+    for (const void *t : {p.u, p.delta, p.z, p.B, p.C, static_cast<const void *>(p.out), static_cast<const void *>(p.out_z)})
+        if (reinterpret_cast<uintptr_t>(t) % eb) return false;
+    return p.seqlen >= kMinRagged && p.batch <= 65535 && k2s_bytes_ok(p);
+}
+// Whether the request takes it. Aligned rows keep the buffer-addressed kernels where every tile pair is
+// whole, at 8 and 16 steps (batch 64, 5,120 channels, bf16, L 8: 64 us against 88 us), and where a
+// variant is forced for measurements.
+static bool ragged_route(const mm_scan_fwd_params &p) {
+    if (!ragged_ok(p)) return false;
+    const bool aligned = fwd_vector_ok(&p) && tiled_shape_ok(p);
+    return !aligned || !(p.seqlen % (2 * tiled::kT1) == 0 || p.seqlen <= tiled::kT1 || tiled_variant() != 0);
+}
+
 // Whether a segmented request runs on k2s: every 32-step pair whole, byte offsets in range, and
 // neither a request that writes both out and out_z nor fp32 with chunk states (the pipelined
 // kernel's segments serve those; MM_SCAN_KERNEL=k2 selects them always).
@@ -1815,7 +1929,7 @@ int64_t device_simds() {
 // (6, 8) cost most, and from ~5 waves per SIMD on the time is flat. MM_SCAN_SEGMENTS=n sets the count
 // (for measurements).
 int64_t segment_count(const mm_scan_fwd_params &p) {
-    if (!tiled_shape_ok(p) || !fwd_vector_ok(&p) || !pipe_offsets_ok(p) || p.tile_states) return 1;
+    if (!ragged_route(p) && (!tiled_shape_ok(p) || !fwd_vector_ok(&p) || !pipe_offsets_ok(p) || p.tile_states)) return 1;
     const int64_t waves = 2 * p.batch * (p.dim / tiled::kCh);
     const int64_t n_pairs = (p.seqlen + 2 * tiled::kT1 - 1) / (2 * tiled::kT1);
     int64_t n_seg;
@@ -1898,8 +2012,9 @@ static int launch_k2x(const mm_scan_fwd_params &p, hipStream_t stream) {
 
 template <typename T>
 int try_launch_tiled(const mm_scan_fwd_params &p, hipStream_t stream) {
-    if (!tiled_shape_ok(p) || !fwd_vector_ok(&p)) return MM_ERR_UNSUPPORTED;
-    const bool pipe_ok = pipe_offsets_ok(p);
+    const bool ragged = ragged_route(p);
+    if (!ragged && (!tiled_shape_ok(p) || !fwd_vector_ok(&p))) return MM_ERR_UNSUPPORTED;
+    const bool pipe_ok = ragged || pipe_offsets_ok(p);
     if (p.tile_states) {
         // The backward's checkpoints are written by the default kernels only (one pass, no segments).
         if (!pipe_ok) return MM_ERR_UNSUPPORTED;
@@ -1914,12 +2029,14 @@ int try_launch_tiled(const mm_scan_fwd_params &p, hipStream_t stream) {
         float *ws = static_cast<float *>(p.workspace);
         const tiled::SegArgs sg{(n_pairs + n_seg - 1) / n_seg, int32_t(n_seg), ws, ws + rows * n_seg * 16,
                                 ws + rows * n_seg * 17};
+        if (ragged) return tiled::launch_k2s_ragged<T>(p, stream, sg);
         if (k2s_segments_ok(p)) {
             const int rc = tiled::launch_k2s_segmented<T>(p, stream, sg);
             if (rc != MM_ERR_UNSUPPORTED) return rc;
         }
         return tiled::launch_pipe_segmented<T>(p, stream, sg);
     }
+    if (ragged) return tiled::launch_k2s_ragged<T>(p, stream, tiled::kWholeRows);
     switch (pipe_ok ? tiled_variant() : 2) {
         case 1: return tiled::launch_nw<T, 1>(p, stream);
         case 2: return tiled::launch_nw<T, 2>(p, stream);

@@ -27,11 +27,10 @@ included), which is what the reference returns in both of its gradient modes
 through its torch loop (calls with z) differentiate the same function; "exact" takes dP/dQ of
 z-less calls from that autograd, any other value ("fused") from the dense kernel, the only backward
 its launcher runs with P/Q (selective_scan_bwd_kernel.cuh:928-932), which accumulates the same
-chain rule (:307, :334). The variable is therefore not read here. The fast gfx950 backward covers
-pq_rank 1..8, dstate <= 16, dim and dim / n_groups multiples of 16 and seqlen a multiple of 8, with
-variable B and C; training requests of other lengths are padded in front with zero-u steps
-(_train_pad); the other shapes the reference takes (dstate <= 256, rank <= 8, constant B or C) run
-a general P/Q backward with one lane per state.
+chain rule (:307, :334). The variable is therefore not read here. One gfx950 kernel covers dstate <= 64 (pq_rank 1..8, 1..4
+past dstate 32) with variable B and C, dim and dim / n_groups multiples of 16 and any seqlen; the
+other shapes the reference takes (dstate <= 256, rank <= 8, constant B or C) run a general P/Q
+backward with one lane per state.
 
 Differences (all raise instead of computing something else): complex A is not part of this build.
 """
@@ -53,20 +52,17 @@ def _save_tile_states():
 
 
 def _train_pad(u, A, B, C):
-    """Steps to put in front of a training request whose length is not a multiple of 8, so that
-    the forward and backward run the fast kernels (the diagonal ones at dstate 16, the P/Q ones at
-    dstate <= 16, which also run the diagonal scan at other dstate values with a zero coupling;
-    with other lengths the diagonal scan would run the general kernels, ~14x and ~100x slower, and
-    the P/Q backward would refuse the call). The padded steps carry zero u, delta, z, B and C, and
-    dout is zero over them: from the zero initial state a zero-u step leaves every state exactly
-    zero, so the real steps run the unpadded recurrence, and the padded steps add nothing to dA,
-    dD, ddelta_bias, dP or dQ (each of their terms holds u, h or Q h of a padded step). 0 when no
-    padding applies, or with MM_SCAN_PAD=0 (which also turns off the binding's padding of
-    inference requests)."""
+    """Steps to put in front of a diagonal training request at dstate 16 whose length is not a
+    multiple of 8, so that its forward runs the kernels that write the tile states and its backward
+    the dstate-16 one (the other requests' kernels take any length). The padded steps carry zero u,
+    delta, z, B and C, and dout is zero over them: from the zero initial state a zero-u step leaves
+    every state exactly zero, so the real steps run the unpadded recurrence, and the padded steps add
+    nothing to dA, dD or ddelta_bias (each of their terms holds u or h of a padded step). 0 when no
+    padding applies, or with MM_SCAN_PAD=0."""
     L = u.shape[-1]
     if L % 8 == 0 or B.dim() != 4 or C.dim() != 4 or os.environ.get("MM_SCAN_PAD", "1") == "0":
         return 0
-    if A.shape[1] > 16:
+    if A.shape[1] != 16:
         return 0
     dim, groups = u.shape[1], B.shape[1]
     if dim % 16 or (dim // groups) % 16:
@@ -219,8 +215,6 @@ class SelectiveScanPQFn(torch.autograd.Function):
         # dstate <= 16 the forward also writes the states before every 16-step tile (B * dim * L
         # float32, about one float32 copy of u), which spare the backward a recompute of the scan.
         want_ck = A.shape[1] <= 16 and P.shape[-1] > 0 and _save_tile_states()
-        pad = ctx.pad = _train_pad(u, A, B, C)
-        u, delta, z, B, C = (_pad_front(t, pad) for t in (u, delta, z, B, C))
         out, x, *rest = ext().fwd(u, delta, A, B, C, D, z, delta_bias, P, Q, gamma, delta_softplus,
                                   tile_states=want_ck)
         ck = rest.pop() if want_ck else None
@@ -230,7 +224,6 @@ class SelectiveScanPQFn(torch.autograd.Function):
                               out if ctx.has_z else None, ck)
         last_state = x[:, :, -1, 1::2]
         result = rest[0] if ctx.has_z else out
-        result = _unpad(result, pad).contiguous() if pad else result
         return result if not return_last_state else (result, last_state)
 
     @staticmethod
@@ -242,8 +235,6 @@ class SelectiveScanPQFn(torch.autograd.Function):
         u, delta, A, B, C, D, z, delta_bias, P, Q, gamma, x, out, ck = ctx.saved_tensors
         if dout.stride(-1) != 1:
             dout = dout.contiguous()
-        pad = ctx.pad
-        dout = _pad_front(dout, pad)
         dP = torch.zeros(P.shape, dtype=torch.float32, device=P.device)
         dQ = torch.zeros(Q.shape, dtype=torch.float32, device=Q.device)
         du, ddelta, dA, dB, dC, dD, ddelta_bias, *rest = ext().bwd(
@@ -251,7 +242,6 @@ class SelectiveScanPQFn(torch.autograd.Function):
             x=x, out=out, dz=None, dP_out=dP, dQ_out=dQ, delta_softplus=ctx.delta_softplus,
             recompute_out_z=False, tile_states=ck)
         dz = rest[0] if ctx.has_z else None
-        du, ddelta, dz, dB, dC = (_unpad(t, pad) for t in (du, ddelta, dz, dB, dC))
         dB = dB.squeeze(1) if getattr(ctx, "squeeze_B", False) else dB
         dC = dC.squeeze(1) if getattr(ctx, "squeeze_C", False) else dC
         return (du, ddelta, dA, dB, dC,
