@@ -138,7 +138,7 @@ typedef struct mm_scan_fwd_params {
      * B * dim * seqlen * 4 bytes, about one float32 copy of u. Passed to mm_scan_bwd as
      * `tile_states`, they spare it the recompute of the whole forward. Written with P/Q and
      * dstate <= 16, and without P/Q together with chunk_states (the training forward) by the
-     * dstate-16 kernels or, below dstate 16, the P/Q kernels run with a zero coupling
+     * dstate-16 kernels or, below dstate 16, the P/Q kernels without a coupling
      * (mm_scan_fwd_tile_states_size() is non-zero exactly when this request can write them).
      * NULL: not written. */
     float *tile_states;

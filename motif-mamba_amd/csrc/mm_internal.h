@@ -39,14 +39,12 @@ int64_t device_simds();
 // Forward scan with the low-rank P/Q coupling (mm_scan_pq.hip): the tiled kernel when the request
 // fits it, else the lane-per-row kernel.
 template <typename T>
-int launch_pq(const mm_scan_fwd_params &p, hipStream_t stream, bool diag_x = false);
+int launch_pq(const mm_scan_fwd_params &p, hipStream_t stream);
 
-// The diagonal scan on the P/Q kernels (mm_scan_pq.hip), for requests the dstate-16 kernels do not
-// take: diag_via_pq_fwd tells whether a forward goes that way (dstate != 16 up to 64) with the zero
-// rank-1 pair that attach_zero_pair puts in a copy of its parameters, diag_lanes_bwd whether a
-// backward (dstate <= 64) runs scan_bwd_lanes without a coupling.
+// The diagonal scan on the P/Q kernels without a coupling, for requests the dstate-16 kernels do not
+// take: diag_via_pq_fwd tells whether a forward goes that way (dstate != 16 up to 64, launch_pq then
+// takes it), diag_lanes_bwd whether a backward does (dstate <= 64, scan_bwd_lanes).
 bool diag_via_pq_fwd(const mm_scan_fwd_params &p);
-int attach_zero_pair(mm_scan_fwd_params &q);
 bool diag_lanes_bwd(const mm_scan_bwd_params &p);
 
 // Backward (mm_scan_bwd.hip): clears the accumulated gradients and launches the backward kernels

@@ -572,7 +572,7 @@ int validate_fwd(const mm_scan_fwd_params *p) {
                                              "(the training forward)");
     if (p->tile_states && !p->P && !mm::tile_states_ok(*p) && !mm::diag_via_pq_fwd(*p))
         return fail(MM_ERR_UNSUPPORTED, "mm_scan_fwd: without P/Q, tile_states are written by the dstate-16 kernels "
-                                        "and, below dstate 16, by the P/Q kernels with a zero coupling (variable "
+                                        "and, below dstate 16, by the P/Q kernels without a coupling (variable "
                                         "B/C, dim and dim / n_groups multiples of 16, L a multiple of 8, aligned "
                                         "rows); mm_scan_fwd_tile_states_size tells");
     return MM_OK;
@@ -602,11 +602,7 @@ int launch_rowlane(const mm_scan_fwd_params &p, hipStream_t s) {
 
 template <typename T>
 int dispatch_fwd(const mm_scan_fwd_params &p, hipStream_t s) {
-    if (p.P) return mm::launch_pq<T>(p, s);
-    if (mm::diag_via_pq_fwd(p)) {
-        mm_scan_fwd_params q = p;
-        if (mm::attach_zero_pair(q) == MM_OK) return mm::launch_pq<T>(q, s, true);
-    }
+    if (p.P || mm::diag_via_pq_fwd(p)) return mm::launch_pq<T>(p, s);
     int rc = mm::try_launch_tiled<T>(p, s);
     if (rc != MM_ERR_UNSUPPORTED || p.tile_states) return rc;   // the general kernel writes no tile states
     return launch_rowlane<T>(p, s);

@@ -38,7 +38,6 @@
 #include <stdlib.h>
 
 #include <algorithm>
-#include <atomic>
 
 #include <type_traits>
 
@@ -72,15 +71,19 @@ __device__ __forceinline__ void lds_read_vec(const float *src, float *o) {
     }
 }
 
-// DX: the chunk states in the diagonal scan's form, (prod of the decays since step 0, h), for the
-// diagonal requests run with a zero P/Q pair; otherwise (1, h), the P/Q form.
+// R = 0: no coupling, the diagonal scan of the dstate values the dstate-16 kernels do not take, with
+// the chunk states in its form, (prod of the decays since step 0, h); otherwise (1, h), the P/Q form.
+// 8 x 1,536 channels, L 1,024, bf16, dstate 64: 0.436 -> 0.287 ms against the rank-2 instance with a
+// zero pair; 4 x 2,048 channels, L 2,048, dstate 32: 0.28 -> 0.18 ms, dstate 8: 0.20 -> 0.14 ms.
 // VEC: every row starts 16-byte aligned and L is a multiple of 8. Without it (any L, any row
 // alignment) the same vectors move through global accesses that need only the element's alignment,
 // and the last, partial tile moves element by element: 3 x 4,320 channels, L 1,797, dstate 16, rank
 // 2, fp16 0.25 ms against 0.45 ms on copies padded to whole tiles.
-template <typename T, int S, int LPR, int R, bool DX = false, bool VEC = true>
+template <typename T, int S, int LPR, int R, bool VEC = true>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t blocks_per_group) {
+    constexpr bool DX = R == 0;
+    constexpr int RR = R > 0 ? R : 1;
     constexpr int NP = S * LPR;            // padded states per channel
     constexpr int CPW = 64 / LPR;          // channels per wave
     constexpr int E = kT / LPR;            // prologue / epilogue steps per lane per tile
@@ -117,11 +120,11 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     // XK: the carried form described below. TS: the coupling's R sums over the channel's lanes are one transposed
     // reduction (lane_sums, R <= LPR), which wants the lane's rows of Q and columns of P in its
     // order: position t holds rank t ^ ro.
-    constexpr bool XK = LPR == 16 && S == 1 && R <= 2 && !std::is_same<T, float>::value;
-    constexpr bool TS = R <= LPR && !XK;
+    constexpr bool XK = LPR == 16 && S == 1 && R > 0 && R <= 2 && !std::is_same<T, float>::value;
+    constexpr bool TS = R > 0 && R <= LPR && !XK;
     int ro = 0;
     if constexpr (TS) ro = lane_rank_offset<LPR, R>(k);
-    float A2[S], h[S], Pr[S][R], Qr[R][S];
+    float A2[S], h[S], Pr[S][RR], Qr[RR][S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int n = k * S + s;
@@ -146,7 +149,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     // chain); +10 % at two waves per SIMD with 8 lanes, where issue sets the time. 16-bit inputs
     // only: float32 callers keep the direct Q h, whose rounding the long-sequence float32 checks
     // pin; 16-bit outputs round far above the float32 rounding difference of the two forms.
-    float Kr[R][R], gq[R];
+    float Kr[RR][RR], gq[RR];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         gq[r] = 0.f;
@@ -163,7 +166,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     const bool softplus = p.delta_softplus != 0;
     const int es = E * k;                  // first step (within a tile) of this lane's elements
     const int64_t n_chunks = (L + MM_SCAN_CHUNK - 1) / MM_SCAN_CHUNK;
-    float cum_dt = 0.f;                    // DX: running sum of dt' (prod a = exp2(A log2e cum_dt))
+    float cum_dt = 0.f;                    // R = 0: running sum of dt' (prod a = exp2(A log2e cum_dt))
     // Checkpoints for the backward: the S states of this lane before every 16-step tile.
     const int64_t ck_tile = p.batch * p.dim * 16;
     float *const ckp = (p.tile_states && active) ? p.tile_states + (b * p.dim + d) * 16 + k * S : nullptr;
@@ -414,7 +417,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float q[R], y = 0.f;
+                float q[RR], y = 0.f;
                 if constexpr (XK) {
                     // h_t = hb + P q with hb = a h_{t-1} + dt' u B and q = dt' gq; the next step's
                     // lane partial of Q h_t as X + K q, where X = Q hb needs only h_{t-1} (off the
@@ -935,35 +938,38 @@ static TiledShape tiled_shape(const mm_scan_fwd_params &p) {
     // per SIMD; dstate 32: 0.60 against 0.47 ms at 1.5). At dstate 16, 8 lanes of 2 states stay the
     // fastest up to 2.5 of their waves per SIMD (0.30 ms at two, 0.40 ms at 2.5 against 0.45 ms with
     // 4 lanes); past that the 4-lane layout's half as many waves win (0.45 against 0.55 ms at 3).
+    // Without a coupling the lanes of a channel only meet in y: bf16, L 2048, 2,048 channels x batch 4
+    // (1,024 waves of 8 lanes): 0.183 against 0.199 ms at dstate 32, equal at dstate 8; with 1,536 such
+    // waves 0.150 against 0.138 and 0.134 against 0.094 ms, and 4 lanes stay behind 8 (dstate 8, 2,560
+    // waves of 8: 0.296 against 0.244 ms).
     const int64_t simds = device_simds();
     if (nc == 1) return cands[0];
+    if (!p.P) return waves(16) <= 2 * simds ? cands[nc - 1] : (nc == 3 ? cands[1] : cands[0]);
     if (waves(16) <= simds) return cands[nc - 1];
     if (nc == 2) return cands[0];
     return 2 * waves(8) <= 5 * simds ? cands[1] : cands[0];
 }
 
-template <typename T, int S, int LPR, int R, bool DX, bool VEC>
+template <typename T, int S, int LPR, int R, bool VEC>
 int launch_tiled_sr(const mm_scan_fwd_params &p, hipStream_t s) {
     constexpr int CPW = 64 / LPR;
     const int64_t ratio = p.dim / p.n_groups;
     const int64_t bpg = (ratio + CPW - 1) / CPW;
     dim3 grid(unsigned(bpg * p.n_groups), unsigned(p.batch));
-    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, DX, VEC>), grid, dim3(64), 0, s, p, ratio, int32_t(bpg));
+    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, VEC>), grid, dim3(64), 0, s, p, ratio, int32_t(bpg));
     return launch_status("scan_fwd_pq_tiled");
 }
 
-// diag_x: the zero-pair diagonal route, which has rank 1 and wants the diagonal chunk states.
 template <typename T, int S, int LPR, bool VEC>
-int launch_tiled_v(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
-    if (diag_x) return launch_tiled_sr<T, S, LPR, 2, true, VEC>(p, s);
-    if (p.pq_rank <= 2) return launch_tiled_sr<T, S, LPR, 2, false, VEC>(p, s);
-    if (p.pq_rank <= 4) return launch_tiled_sr<T, S, LPR, 4, false, VEC>(p, s);
-    return launch_tiled_sr<T, S, LPR, 8, false, VEC>(p, s);
+int launch_tiled_v(const mm_scan_fwd_params &p, hipStream_t s) {
+    if (!p.P) return launch_tiled_sr<T, S, LPR, 0, VEC>(p, s);
+    if (p.pq_rank <= 2) return launch_tiled_sr<T, S, LPR, 2, VEC>(p, s);
+    if (p.pq_rank <= 4) return launch_tiled_sr<T, S, LPR, 4, VEC>(p, s);
+    return launch_tiled_sr<T, S, LPR, 8, VEC>(p, s);
 }
 template <typename T, int S, int LPR>
-int launch_tiled_s(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
-    return fwd_vector_ok(&p) ? launch_tiled_v<T, S, LPR, true>(p, s, diag_x)
-                             : launch_tiled_v<T, S, LPR, false>(p, s, diag_x);
+int launch_tiled_s(const mm_scan_fwd_params &p, hipStream_t s) {
+    return fwd_vector_ok(&p) ? launch_tiled_v<T, S, LPR, true>(p, s) : launch_tiled_v<T, S, LPR, false>(p, s);
 }
 
 // One-step requests with variable B and C that write no chunk or tile states take the step kernel:
@@ -1006,50 +1012,27 @@ int launch_rowlane(const mm_scan_fwd_params &p, hipStream_t s) {
 }  // namespace pq
 
 template <typename T>
-int launch_pq(const mm_scan_fwd_params &p, hipStream_t s, bool diag_x) {
+int launch_pq(const mm_scan_fwd_params &p, hipStream_t s) {
     const pq::TiledShape sh = pq::tiled_shape(p);
-    if (sh.LPR == 4) return pq::launch_tiled_s<T, 4, 4>(p, s, diag_x);
-    if (sh.LPR == 8)
-        return sh.S == 4 ? pq::launch_tiled_s<T, 4, 8>(p, s, diag_x) : pq::launch_tiled_s<T, 2, 8>(p, s, diag_x);
+    if (sh.LPR == 4) return pq::launch_tiled_s<T, 4, 4>(p, s);
+    if (sh.LPR == 8) return sh.S == 4 ? pq::launch_tiled_s<T, 4, 8>(p, s) : pq::launch_tiled_s<T, 2, 8>(p, s);
     if (sh.LPR == 16) {
-        if (sh.S == 4) return pq::launch_tiled_s<T, 4, 16>(p, s, diag_x);
-        if (sh.S == 2) return pq::launch_tiled_s<T, 2, 16>(p, s, diag_x);
-        return pq::launch_tiled_s<T, 1, 16>(p, s, diag_x);
+        if (sh.S == 4) return pq::launch_tiled_s<T, 4, 16>(p, s);
+        if (sh.S == 2) return pq::launch_tiled_s<T, 2, 16>(p, s);
+        return pq::launch_tiled_s<T, 1, 16>(p, s);
     }
-    return pq::launch_rowlane<T>(p, s);   // not reached with diag_x (diag_via_pq_fwd requires a tiled shape)
+    return pq::launch_rowlane<T>(p, s);   // with P and Q (diag_via_pq_fwd requires a tiled shape)
 }
 
-template int launch_pq<MM_PQ_TYPE>(const mm_scan_fwd_params &, hipStream_t, bool);
+template int launch_pq<MM_PQ_TYPE>(const mm_scan_fwd_params &, hipStream_t);
 
 #ifdef MM_PQ_COMMON
 
 // ------------------------------------------------------------------------------------------------
-// The diagonal scan through the P/Q kernels. A zero rank-1 pair shared by every channel (P = Q = 0)
-// leaves the coupled recurrence exactly the diagonal one: q = Q h = 0 and every coupling term is
-// fma(0, q, w) = w. Diagonal forwards the dstate-16 kernels do not take (dstate below 16, or 17 to
-// 64, variable B and C) run several times faster this way than on the general kernels. The pair is a
-// static device array; its address is looked up once per device. Diagonal backwards that the
-// dstate-16 kernel does not take run the P/Q backward's instance without a coupling.
+// The diagonal scan on the P/Q kernels without a coupling: requests the dstate-16 kernels do not take
+// (forwards with dstate below 16, or 17 to 64; backwards also of odd lengths and unaligned rows), variable
+// B and C, run several times faster this way than on the general kernels.
 namespace {
-__device__ __align__(16) float pq_zero_pair[64];   // zero-initialised, never written
-
-constexpr int kMaxDev = 64;
-std::atomic<float *> g_zero_ptr[kMaxDev];
-
-int zero_pair_pointer(float **zero) {
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return MM_ERR_UNSUPPORTED;
-    float *z = g_zero_ptr[dev].load(std::memory_order_acquire);
-    if (z == nullptr) {
-        void *a = nullptr;
-        if (hipGetSymbolAddress(&a, HIP_SYMBOL(pq_zero_pair)) != hipSuccess || a == nullptr) return MM_ERR_UNSUPPORTED;
-        z = static_cast<float *>(a);
-        g_zero_ptr[dev].store(z, std::memory_order_release);
-    }
-    *zero = z;
-    return MM_OK;
-}
-
 // MM_DIAG_VIA_PQ=0 keeps such requests on the general kernels (read per call, for the tests).
 bool diag_pq_enabled() {
     const char *e = getenv("MM_DIAG_VIA_PQ");
@@ -1063,19 +1046,6 @@ bool diag_via_pq_fwd(const mm_scan_fwd_params &p) {
     if (p.P || p.dstate == 16 || p.dstate > 64 || (p.tile_states && p.dstate > 16) || !diag_pq_enabled())
         return false;
     return pq::tiled_shape(p).LPR != 0;
-}
-
-int attach_zero_pair(mm_scan_fwd_params &q) {
-    float *zero = nullptr;
-    const int rc = zero_pair_pointer(&zero);
-    if (rc != MM_OK) return rc;
-    q.P = zero;
-    q.Q = zero;
-    q.gamma = nullptr;
-    q.pq_rank = 1;
-    q.P_d_stride = 0; q.P_dstate_stride = 1; q.P_r_stride = 0;
-    q.Q_d_stride = 0; q.Q_r_stride = 0; q.Q_dstate_stride = 1;
-    return MM_OK;
 }
 
 bool diag_lanes_bwd(const mm_scan_bwd_params &p) {
