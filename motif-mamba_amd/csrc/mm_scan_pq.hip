@@ -11,8 +11,8 @@
 // set of independent per-state scans: each state needs Q h_{t-1} before it can take step t. The
 // design of this file is its own:
 //
-//   scan_fwd_pq_tiled<T, S, LPR, R>   a wave64 owns 64/LPR channels of one (batch, group); the LPR
-//       consecutive lanes of a channel hold S states each (S * LPR >= dstate, padded with states
+//   scan_fwd_pq_tiled<T, S, LPR, R>   a wave64 owns 64/LPR channels of one (batch, group), at
+//       dstate above 32 four of them in a workgroup; the LPR consecutive lanes of a channel hold S states each (S * LPR >= dstate, padded with states
 //       whose A, P, Q, B and C are zero, which stay zero). Per step each lane forms its partial
 //       Q h over its S states, a DPP butterfly inside the LPR lanes sums the partials (every lane
 //       ends with the same bits; where the rank is at most LPR one transposed butterfly serves all
@@ -71,6 +71,19 @@ __device__ __forceinline__ void lds_read_vec(const float *src, float *o) {
     }
 }
 
+// Waves per workgroup that share the staged B and C. At dstate above 32 a lane alone would load and stage
+// four vectors of each per tile, more than the registers hold beside the scan; four waves take one each
+// (16 channels: 8 x 2,048 channels, L 2,048, bf16, dstate 64: 0.77 -> 0.53 ms, with P/Q of rank 2 at batch 4
+// 0.71 -> 0.43 ms). At dstate 32 two waves would land on the same SIMDs where the grid fills each once
+// (P/Q, 4 x 2,048 channels, L 2,047: 0.28 against 0.43 ms).
+constexpr int waves_sharing(int np) { return np > 32 ? 4 : 1; }
+
+template <typename T, int N>
+__device__ __forceinline__ void pin_raw(RawVec<T, N> &r) {
+#pragma unroll
+    for (auto &w : r.w) asm volatile("" : "+v"(w));
+}
+
 // R = 0: no coupling, the diagonal scan of the dstate values the dstate-16 kernels do not take, with
 // the chunk states in its form, (prod of the decays since step 0, h); otherwise (1, h), the P/Q form.
 // 8 x 1,536 channels, L 1,024, bf16, dstate 64: 0.436 -> 0.287 ms against the rank-2 instance with a
@@ -80,33 +93,35 @@ __device__ __forceinline__ void lds_read_vec(const float *src, float *o) {
 // and the last, partial tile moves element by element: 3 x 4,320 channels, L 1,797, dstate 16, rank
 // 2, fp16 0.25 ms against 0.45 ms on copies padded to whole tiles.
 template <typename T, int S, int LPR, int R, bool VEC = true>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * waves_sharing(S * LPR)) __attribute__((amdgpu_waves_per_eu(2)))
 scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t blocks_per_group) {
     constexpr bool DX = R == 0;
     constexpr int RR = R > 0 ? R : 1;
     constexpr int NP = S * LPR;            // padded states per channel
     constexpr int CPW = 64 / LPR;          // channels per wave
+    constexpr int W = waves_sharing(NP);   // waves per workgroup, sharing the staged B and C
+    constexpr int NU = NP / 16 / W;        // units of B and C a lane stages per tile
     constexpr int E = kT / LPR;            // prologue / epilogue steps per lane per tile
     // sBC row stride (floats): NP B values, then NP C values. The staging writes, for one element
     // position, lanes (state n = lane / 4, step block q = lane % 4) at q 8 BCS + n: with BCS = 2 NP + 2
     // (S <= 2; the scan reads S-vectors of 8 bytes) 8 BCS = 16 mod 64, so the 64 lanes cover 64
     // consecutive banks; S = 4 needs 16-byte aligned rows (2 NP + 4).
     constexpr int BCS = S <= 2 ? 2 * NP + 2 : 2 * NP + 4;
-    constexpr int HR = NP / 16;            // B/C half-rows (16 steps of one state) staged per lane
-    static_assert(HR >= 1 && E >= 2 && E % 2 == 0 && 2 * CPW <= 64, "tile shape");
+    static_assert(NU >= 1 && E >= 2 && E % 2 == 0 && 2 * CPW <= 64, "tile shape");
     __shared__ __align__(16) float sBC[kT * BCS];
-    // During the scan: dt' rows then dt'u rows of the wave's channels; after it: the y partials.
-    __shared__ __align__(16) float sX[64 * kPad];
-    float *sDt = sX;
-    float *sDu = sX + CPW * kPad;
-    float *sY = sX;
+    // Per wave, during the scan: dt' rows then dt'u rows of its channels; after it: the y partials.
+    __shared__ __align__(16) float sX[W * 64 * kPad];
+    const int wave = threadIdx.x / 64;
+    float *sDt = sX + wave * (64 * kPad);
+    float *sDu = sDt + CPW * kPad;
+    float *sY = sDt;
 
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % 64;
     const int cw = lane / LPR;             // channel slot in the wave
     const int k = lane % LPR;              // state slice: states k S .. k S + S - 1
     const int64_t b = blockIdx.y;
     const int64_t g = blockIdx.x / blocks_per_group;
-    const int64_t cl = int64_t(blockIdx.x % blocks_per_group) * CPW + cw;  // channel within the group
+    const int64_t cl = int64_t(blockIdx.x % blocks_per_group) * (CPW * W) + wave * CPW + cw;  // channel within the group
     const bool active = cl < ratio;
     const int64_t d = g * ratio + (active ? cl : ratio - 1);  // inactive slots mirror a real channel
     const int64_t L = p.seqlen;
@@ -175,14 +190,14 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         for (int s = 0; s < S; ++s) ckp[j * ck_tile + s] = h[s];
     };
 
-    // The loads of u, delta and z go through buffer resources: the rows of the wave's channels from
+    // The loads of u, delta and z go through buffer resources: the rows of the workgroup's channels from
     // its first channel dw, with 32-bit byte offsets per lane (the host checks that every offset of
     // these rows fits). A whole tile adds its start as a scalar offset; only the last, partial
     // tile clamps per lane. (B and C, a tensor per lane, keep per-lane pointers: a resource
     // descriptor must be uniform.)
     constexpr uint32_t SZ = sizeof(T);
-    const int64_t dw = g * ratio + int64_t(blockIdx.x % blocks_per_group) * CPW;
-    const int64_t dl = d - dw;             // 0 .. CPW - 1 (inactive slots mirror the group's last channel)
+    const int64_t dw = g * ratio + int64_t(blockIdx.x % blocks_per_group) * (CPW * W);
+    const int64_t dl = d - dw;             // 0 .. CPW W - 1 (inactive slots mirror the group's last channel)
     const __amdgpu_buffer_rsrc_t rs_u = buffer_rsrc(reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride + dw * p.u_d_stride);
     const __amdgpu_buffer_rsrc_t rs_d =
         buffer_rsrc(reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride + dw * p.delta_d_stride);
@@ -198,27 +213,23 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     const uint32_t fo_o = uint32_t(dl * p.out_d_stride + es) * SZ, fo_oz = uint32_t(dl * p.out_z_d_stride + es) * SZ;
 
     // B and C of the (batch, group) through buffer resources too. Per 32-step tile every lane stages
-    // NU = NP / 16 units of each tensor: unit u = lane + 64 i is the 8 steps 8 (u % 4) .. + 7 of
-    // state u / 4, one 8-element load from B and one from C (a 32-bit offset per lane, the tile
-    // start as a scalar offset). Units of padded states (u / 4 >= dstate) and, in a last partial
-    // tile, units past L (L is a multiple of 8: a unit is all in or all out) are zeroed once when
-    // loaded, so the staging below writes every unit unconditionally.
-    constexpr int NU = NP / 16;
+    // NU units of each tensor: unit u is the 8 steps 8 (u % 4) .. + 7 of state u / 4, thread t of the
+    // 64 W takes units t + 64 W i (4 NP in all): one 8-element load from B and one from C each (a 32-bit
+    // offset per lane, the tile start as a scalar offset). Units of padded states (u / 4 >= dstate)
+    // and, in a last partial tile, units past L (L is a multiple of 8: a unit is all in or all out)
+    // are zeroed once when loaded, so the staging below writes every unit unconditionally.
     const __amdgpu_buffer_rsrc_t rs_B = buffer_rsrc(Bg), rs_C = buffer_rsrc(Cg);
-    uint32_t fo_B[NU], fo_C[NU];
-    int u_lds[NU], u_q[NU];
+    const int u_n = threadIdx.x / 4, u_q = threadIdx.x % 4;
     bool u_on[NU];
+    uint32_t fo_B[NU], fo_C[NU];
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-        const int u = lane + 64 * i;
-        const int n = u / 4;
-        u_q[i] = u % 4;
+        const int n = u_n + 16 * W * i;
         u_on[i] = n < N;
-        const int64_t nn = n < N ? n : 0;
-        fo_B[i] = uint32_t(nn * p.B_dstate_stride) * SZ;
-        fo_C[i] = uint32_t(nn * p.C_dstate_stride) * SZ;
-        u_lds[i] = 8 * u_q[i] * BCS + n;
+        fo_B[i] = uint32_t((u_on[i] ? n : 0) * p.B_dstate_stride) * SZ;
+        fo_C[i] = uint32_t((u_on[i] ? n : 0) * p.C_dstate_stride) * SZ;
     }
+    const int u_lds = 8 * u_q * BCS + u_n;
     const bool padded = N < NP;            // uniform
 
     // Loads at or past the end of a row are redirected into the row's last elements (always in
@@ -276,32 +287,29 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         RawVec<T, 8> b[NU], c[NU];
     };
     auto load_bc = [&](int64_t t0, BCs &r) {
-        if constexpr (!VEC) {
-            if (t0 + kT <= L) {            // uniform: a whole tile
-                const int64_t so = t0 * SZ;
+        if (t0 + kT <= L) {                // uniform: a whole tile
 #pragma unroll
-                for (int i = 0; i < NU; ++i) {
-                    r.b[i] = load_any<T, 8>(Bb + so, fo_B[i] + uint32_t(8 * u_q[i]) * SZ);
-                    r.c[i] = load_any<T, 8>(Cb + so, fo_C[i] + uint32_t(8 * u_q[i]) * SZ);
+            for (int i = 0; i < NU; ++i) {
+                if constexpr (VEC) {
+                    const uint32_t so = uint32_t(t0) * SZ;
+                    r.b[i] = buffer_load_rawn<T, 8>(rs_B, fo_B[i] + uint32_t(8 * u_q) * SZ, so);
+                    r.c[i] = buffer_load_rawn<T, 8>(rs_C, fo_C[i] + uint32_t(8 * u_q) * SZ, so);
+                } else {
+                    const int64_t so = t0 * SZ;
+                    r.b[i] = load_any<T, 8>(Bb + so, fo_B[i] + uint32_t(8 * u_q) * SZ);
+                    r.c[i] = load_any<T, 8>(Cb + so, fo_C[i] + uint32_t(8 * u_q) * SZ);
                 }
-            }                              // the last, partial tile: stage_bc loads it
-        } else if (t0 + kT <= L) {         // uniform: a whole tile
-            const uint32_t so = uint32_t(t0) * SZ;
-#pragma unroll
-            for (int i = 0; i < NU; ++i) {
-                r.b[i] = buffer_load_rawn<T, 8>(rs_B, fo_B[i] + uint32_t(8 * u_q[i]) * SZ, so);
-                r.c[i] = buffer_load_rawn<T, 8>(rs_C, fo_C[i] + uint32_t(8 * u_q[i]) * SZ, so);
             }
-        } else {                           // the last, partial tile
+        } else if constexpr (VEC) {        // the last, partial tile
+            const int64_t st = t0 + 8 * u_q;
+            const uint32_t o = uint32_t(st < L ? st : L - 8) * SZ;
 #pragma unroll
             for (int i = 0; i < NU; ++i) {
-                const int64_t st = t0 + 8 * u_q[i];
-                const uint32_t o = uint32_t(st < L ? st : L - 8) * SZ;
                 r.b[i] = buffer_load_rawn<T, 8>(rs_B, fo_B[i] + o, 0);
                 r.c[i] = buffer_load_rawn<T, 8>(rs_C, fo_C[i] + o, 0);
                 if (st >= L) r.b[i] = r.c[i] = {};
             }
-        }
+        }                                  // without VEC stage_bc loads that tile
         if (padded) {
 #pragma unroll
             for (int i = 0; i < NU; ++i)
@@ -311,25 +319,22 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     // Tile rows [step][B states | C states] as float32 (zeros for padded states and past L).
     auto stage_bc = [&](const BCs &r, int64_t t0) {
         if constexpr (!VEC) {
-            if (t0 + kT > L) {             // uniform: the partial tile, element by element, one unit at a time
-#pragma unroll 1
+            if (t0 + kT > L) {             // uniform: the partial tile, element by element
+#pragma unroll
                 for (int i = 0; i < NU; ++i) {
-                    const int u = lane + 64 * i, n = u / 4, q = u % 4;
-                    const uint32_t ob = uint32_t((n < N ? n : 0) * p.B_dstate_stride) * SZ;
-                    const uint32_t oc = uint32_t((n < N ? n : 0) * p.C_dstate_stride) * SZ;
                     uint32_t vb[8], vc[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        const int64_t st = t0 + 8 * q + e;
+                        const int64_t st = t0 + 8 * u_q + e;
                         const uint32_t o = uint32_t(st < L ? st : L - 1) * SZ;
-                        vb[e] = load_elem<T>(Bb, ob + o);
-                        vc[e] = load_elem<T>(Cb, oc + o);
+                        vb[e] = load_elem<T>(Bb, fo_B[i] + o);
+                        vc[e] = load_elem<T>(Cb, fo_C[i] + o);
                     }
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        const bool on = n < N && t0 + 8 * q + e < L;
-                        sBC[(8 * q + e) * BCS + n] = on ? elem_f32<T>(vb[e]) : 0.f;
-                        sBC[(8 * q + e) * BCS + n + NP] = on ? elem_f32<T>(vc[e]) : 0.f;
+                        const bool on = u_on[i] && t0 + 8 * u_q + e < L;
+                        sBC[u_lds + 16 * W * i + e * BCS] = on ? elem_f32<T>(vb[e]) : 0.f;
+                        sBC[u_lds + 16 * W * i + e * BCS + NP] = on ? elem_f32<T>(vc[e]) : 0.f;
                     }
                 }
                 return;
@@ -342,8 +347,20 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
             unpack_raw<T, 8>(r.c[i], vc);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                sBC[u_lds[i] + e * BCS] = vb[e];
-                sBC[u_lds[i] + e * BCS + NP] = vc[e];
+                sBC[u_lds + 16 * W * i + e * BCS] = vb[e];
+                sBC[u_lds + 16 * W * i + e * BCS + NP] = vc[e];
+            }
+        }
+    };
+    auto pin = [&](Elems &e, BCs &r) __attribute__((always_inline)) {
+        pin_raw(e.u);
+        pin_raw(e.d);
+        pin_raw(e.z);
+        if constexpr (!VEC) {
+#pragma unroll
+            for (int i = 0; i < NU; ++i) {
+                pin_raw(r.b[i]);
+                pin_raw(r.c[i]);
             }
         }
     };
@@ -353,11 +370,12 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     if (D == 2) load_elems(kT, e1);
     load_bc(0, b0);
     stage_bc(b0, 0);
+    pin(e0, b0);
     if (D == 2) load_bc(kT, b1);
 
     // Tile t0: its elements in ec, its B/C (already staged) in bc, the next tile's B/C in bn (the
     // same entry as bc when D = 1: loaded at the top of the tile, staged at its end).
-    auto tile = [&](const int64_t t0, Elems &ec, BCs &bc, const BCs &bn) __attribute__((always_inline)) {
+    auto tile = [&](const int64_t t0, Elems &ec, BCs &bc, Elems &en, BCs &bn) __attribute__((always_inline)) {
         const int64_t t1 = t0 + kT;
         // This lane's elements exist: all or none of them where L is a multiple of E.
         auto ev = [&](int i) { return VEC ? t0 + es < L : t0 + es + i < L; };
@@ -491,6 +509,11 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         for (int t = 0; t < kT; t += 4)
             *reinterpret_cast<float4 *>(&sY[(cw * LPR + k) * kPad + t]) = make_float4(yp[t], yp[t + 1], yp[t + 2], yp[t + 3]);
         if (t1 < L) stage_bc(bn, t1);
+        // The next tile's inputs are taken as read here, where they have long arrived: at their first use
+        // (or, B and C, at the next loads into their registers) the wait for them would be one for the
+        // stores below or for the loads just issued as well (2,048 channels, L 30,001, dstate 64, rows of
+        // any alignment: 3.7 -> 2.8 ms).
+        pin(en, bn);
         __syncthreads();
 
         // Epilogue: y of (channel, steps es .. es + E - 1) = the LPR partials, added in lane order.
@@ -548,11 +571,11 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     };
     if constexpr (D == 2) {
         for (int64_t t0 = 0; t0 < L; t0 += 2 * kT) {
-            tile(t0, e0, b0, b1);
-            if (t0 + kT < L) tile(t0 + kT, e1, b1, b0);
+            tile(t0, e0, b0, e1, b1);
+            if (t0 + kT < L) tile(t0 + kT, e1, b1, e0, b0);
         }
     } else {
-        for (int64_t t0 = 0; t0 < L; t0 += kT) tile(t0, e0, b0, b0);
+        for (int64_t t0 = 0; t0 < L; t0 += kT) tile(t0, e0, b0, e0, b0);
     }
     if (active && p.last_state) {
         float *ls = p.last_state + (b * p.dim + d) * N;
@@ -952,11 +975,11 @@ static TiledShape tiled_shape(const mm_scan_fwd_params &p) {
 
 template <typename T, int S, int LPR, int R, bool VEC>
 int launch_tiled_sr(const mm_scan_fwd_params &p, hipStream_t s) {
-    constexpr int CPW = 64 / LPR;
+    constexpr int CPB = 64 / LPR * waves_sharing(S * LPR);   // channels per workgroup
     const int64_t ratio = p.dim / p.n_groups;
-    const int64_t bpg = (ratio + CPW - 1) / CPW;
+    const int64_t bpg = (ratio + CPB - 1) / CPB;
     dim3 grid(unsigned(bpg * p.n_groups), unsigned(p.batch));
-    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, VEC>), grid, dim3(64), 0, s, p, ratio, int32_t(bpg));
+    hipLaunchKernelGGL((scan_fwd_pq_tiled<T, S, LPR, R, VEC>), grid, dim3(64 * waves_sharing(S * LPR)), 0, s, p, ratio, int32_t(bpg));
     return launch_status("scan_fwd_pq_tiled");
 }
 

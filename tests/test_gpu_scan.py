@@ -654,3 +654,17 @@ def test_ragged_rows(L, with_z, dtype):
     out, last = selective_scan_fn(**dev, delta_softplus=True, return_last_state=True)
     torch.cuda.synchronize()
     _rows_vs_f64(dict(host, delta_softplus=True), out.cpu(), last.cpu(), f"ragged L={L}")
+
+
+@pytest.mark.parametrize("N", [17, 32, 33, 64])
+@pytest.mark.parametrize("L", [8, 33, 40])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_shared_tiles_part_filled_workgroups(N, L, dtype):
+    """dstate above 16, where the waves of a workgroup share the staged B and C: channel counts that
+    leave waves of it without a channel, padded states, partial tiles; every row against the float64
+    restatement."""
+    for dim, G in ((1, 1), (9, 1), (17, 1), (34, 2)):
+        _say(f"shared tiles N={N} L={L} dim={dim} G={G} {dtype}")
+        case = _case(170 + N + L, 2, dim, L, N, dtype, bkind="4d", G=G)
+        out, last = _run(case)
+        _rows_vs_f64(case, out, last, f"N={N} dim={dim}")
