@@ -594,16 +594,26 @@ seg_carry_kernel(const float *A, int64_t A_d_stride, int64_t A_dstate_stride, in
     const int n = int(tid & 15);
     const int64_t d = row % dim;
     const float A2 = A[d * A_d_stride + n * A_dstate_stride] * kLog2e;
+    float *const h = sg.h + row * sg.n_seg * 16 + n;
     float H = 0.f, cd = 0.f;
-    for (int s = 0; s < sg.n_seg; ++s) {
-        float *hp = sg.h + (row * sg.n_seg + s) * 16 + n;
-        const bool last = s == sg.n_seg - 1;
-        const float he = last ? 0.f : *hp;
-        const float sd = last ? 0.f : sg.sumdt[row * sg.n_seg + s];
-        *hp = H;
-        if (n == 0) sg.cum[row * sg.n_seg + s] = cd;
-        H = __builtin_fmaf(__builtin_amdgcn_exp2f(A2 * sd), H, he);
-        cd += sd;
+    // A chain of loads, each behind the previous store, would cost a memory latency per segment: eight
+    // segments' values are read at once.
+    for (int s0 = 0; s0 < sg.n_seg; s0 += 8) {
+        float he[8], sd[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const bool on = s0 + i < sg.n_seg - 1;   // nothing follows the last segment
+            he[i] = on ? h[(s0 + i) * 16] : 0.f;
+            sd[i] = on ? sg.sumdt[row * sg.n_seg + s0 + i] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (s0 + i >= sg.n_seg) break;
+            h[(s0 + i) * 16] = H;
+            if (n == 0) sg.cum[row * sg.n_seg + s0 + i] = cd;
+            H = __builtin_fmaf(__builtin_amdgcn_exp2f(A2 * sd[i]), H, he[i]);
+            cd += sd[i];
+        }
     }
 }
 
@@ -1922,12 +1932,15 @@ int64_t device_simds() {
 }
 
 // Sequence segments for shapes whose (batch, 16-channel) groups give fewer than one wave per SIMD
-// (two waves per group): enough segments for ~5 waves per SIMD in the full pass, each at least 512
-// steps. Measured at config 3 (160 groups, L 65,536, fp32, k2s segments): 6, 8, 9, 10, 12, 15, 16,
-// 19, 24 and 32 segments take 1.42, 1.44, 1.31, 1.48, 1.40, 1.29, 1.24, 1.24, 1.25 and 1.25 ms -- a
-// full pass just past one round of workgroups (10, 12) or a few long segments at 2 waves per SIMD
-// (6, 8) cost most, and from ~5 waves per SIMD on the time is flat. MM_SCAN_SEGMENTS=n sets the count
-// (for measurements).
+// (two waves per group), from 512 steps on (256 steps: 14 us whole, 17 to 21 us in 2 to 4 segments).
+// Two plans: as many segments of at least 64 steps as give three waves per SIMD, or of at least 512
+// steps as give five, whichever needs fewer rounds of waves per step of a segment. bf16,
+// against at most five waves per SIMD of at least 512 steps: 512 channels, L 1,024: 46 -> 19 us; 2 x
+// 1,536, L 2,048: 69 -> 58 us (L 1,777: 94 -> 58 us); 5,120, L 1,024: 68 -> 50 us; 3 x 2,560, L 8,192:
+// 434 -> 421 us. From 1,024 waves on whole rows win (2 x 5,120, L 1,024: 70 us, 83 to 91 in segments).
+// Long rows: 160 groups, L 65,536, fp32, 6, 8, 9, 10, 12, 15, 16, 19, 24 and 32 segments take 1.42,
+// 1.44, 1.31, 1.48, 1.40, 1.29, 1.24, 1.24, 1.25 and 1.25 ms. MM_SCAN_SEGMENTS=n sets the count (for
+// measurements).
 int64_t segment_count(const mm_scan_fwd_params &p) {
     if (!ragged_route(p) && (!tiled_shape_ok(p) || !fwd_vector_ok(&p) || !pipe_offsets_ok(p) || p.tile_states)) return 1;
     const int64_t waves = 2 * p.batch * (p.dim / tiled::kCh);
@@ -1937,8 +1950,11 @@ int64_t segment_count(const mm_scan_fwd_params &p) {
         n_seg = std::min<int64_t>(std::atoll(e), n_pairs);
     } else {
         const int64_t simds = device_simds();
-        if (waves >= simds) return 1;
-        n_seg = std::min((5 * simds + waves - 1) / waves, n_pairs / 16);
+        if (waves >= simds || n_pairs < 16) return 1;
+        const int64_t few = std::min(3 * simds / waves, n_pairs / 2);
+        const int64_t many = std::min((5 * simds + waves - 1) / waves, n_pairs / 16);
+        auto rounds = [&](int64_t n) { return (waves * n + simds - 1) / simds; };
+        n_seg = rounds(many) * few < rounds(few) * many ? many : few;
     }
     if (n_seg < 2) return 1;
     const int64_t pairs = (n_pairs + n_seg - 1) / n_seg;

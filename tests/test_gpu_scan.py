@@ -668,3 +668,15 @@ def test_shared_tiles_part_filled_workgroups(N, L, dtype):
         case = _case(170 + N + L, 2, dim, L, N, dtype, bkind="4d", G=G)
         out, last = _run(case)
         _rows_vs_f64(case, out, last, f"N={N} dim={dim}")
+
+
+@pytest.mark.parametrize("n_seg", [2, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("L", [1088, 1001])
+def test_segment_counts(n_seg, L, monkeypatch):
+    """Carry chains around the eight segments read at once (short segments, the last one shorter),
+    whole tiles and ragged rows; every row against the float64 restatement."""
+    monkeypatch.setenv("MM_SCAN_SEGMENTS", str(n_seg))
+    _say(f"segment counts {n_seg} L={L}")
+    case = _case(190 + n_seg, 2, 32, L, 16, torch.bfloat16, bkind="4d", G=1)
+    out, last = _run(case)
+    _rows_vs_f64(case, out, last, f"n_seg={n_seg} L={L}")
