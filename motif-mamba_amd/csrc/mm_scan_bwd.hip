@@ -1305,10 +1305,20 @@ int launch_gen_slab_reduce(const mm_scan_bwd_params &p, hipStream_t s, const flo
     return launch_status("gen_slab_reduce");
 }
 
-bool bwd_tiled_ok(const mm_scan_bwd_params &p) { return bwd::fast_ok(p) || bwd::split_ok(p); }
+// The dstate-16 kernel, or its state split where scan_bwd_lanes is not faster. The split passes over the
+// inputs once per 16 states but can cut rows into sequence segments; from one 16-channel workgroup per CU
+// on scan_bwd_lanes wins at dstate 32 and 64 (bf16: 2 x 2,048 channels, L 2,048: 614 -> 577 and 1,177 ->
+// 935 us; 4 x 5,120, L 2,048: 1.92 -> 1.52 and 3.95 -> 3.50 ms; fp32, 8 x 1,536, L 1,024, dstate 64: 2.40
+// -> 1.12 ms; with 64 workgroups, L 2,048, dstate 32, it loses: 324 against 535 us). At dstate 48 a
+// quarter of its lanes hold padding: 2.94 against 3.38 ms at 4 x 5,120.
+bool bwd_tiled_ok(const mm_scan_bwd_params &p) {
+    if (bwd::fast_ok(p)) return true;
+    return bwd::split_ok(p) && !(bwd_lanes_ok(p) && p.dstate == bwd_lanes_np(p) &&
+                                 4 * p.batch * (p.dim / 16) >= device_simds());
+}
 
 int64_t bwd_workspace_bytes(const mm_scan_bwd_params &p) {
-    if (bwd::split_ok(p))   // one part's workspace (reused by every part), then the carried sums
+    if (!diag_lanes_bwd(p) && bwd::split_ok(p))   // one part's workspace (reused by every part), then the carried sums
         return ((bwd_workspace_bytes(bwd::split_part(p, 0)) + 255) & ~int64_t(255)) +
                bwd::split_acc_floats(p) * int64_t(sizeof(float));
     if (p.P && !bwd_lanes_ok(p))   // the general P/Q backward: its own checkpoints and the slabs

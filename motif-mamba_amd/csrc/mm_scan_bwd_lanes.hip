@@ -22,8 +22,8 @@
 // <= 32, 16 x 4 for <= 64), so that the sums over a channel's states that feed the recurrences (Q h
 // and P^T lam) stay inside 16 lanes: one transposed DPP butterfly each (lane_sums, mm_common.h).
 //
-//   * The kernel is bound by VALU issue (two waves per SIMD, all the registers its tile needs), so
-//     what a step costs is its instruction count. The states and (S = 2, rank <= 4) decays
+//   * The kernel is bound by VALU issue (two waves per SIMD with a coupling, all the registers its tile
+//     needs), so what a step costs is its instruction count. The states and (S = 2, rank <= 4) decays
 //     of a 16-step tile stay in registers between the recompute and the reverse walk; the P q term
 //     of dt' is taken as sum_r q_r (P^T lam)_r from the lane's partials and the u B term as
 //     u_t sum_n lam B by the step's owner, so neither costs a multiply per state.
@@ -32,6 +32,11 @@
 //     butterflies for the sums, took more instructions -- and every lane then finishes one (channel,
 //     step) and one (step, state) of them. The row strides of both keep writes and 16-byte reads at
 //     the LDS's full rate (the dstate 64 layout's dB / dC writes excepted: two-way conflicts).
+//     Without a coupling (rank 0) the dB / dC terms are instead summed over the wave's channels in
+//     registers, by swaps of lane halves and of 16-lane rows that reduce two states of both tensors at
+//     once, and only the waves' sums go through LDS: a third less LDS (23 KB at dstate 16) and no 16-term
+//     sum per row, so three waves per SIMD (8 x 1,536 channels, L 1,024, bf16: 1.63 -> 1.14 ms at dstate
+//     64, 8 x 1,024: 0.43 -> 0.36 ms at dstate 32). With P, Q, dP and dQ the registers lack the room.
 //   * Activations and B / C move one element at a time (uniform row bases, fixed 32-bit
 //     lane offsets), loaded one tile ahead: any length and row alignment, at
 //     about one load per step and lane group.
@@ -71,25 +76,40 @@ constexpr int kT = 16;           // steps per tile
 constexpr int kXS = kT + 1;      // sX row stride (float4)
 constexpr int kRS = kCh + 2;     // sRed row stride (float2)
 
-template <int LPR, int S>
+template <int LPR, int S, int R>
 struct Layout {
+    static constexpr bool SW = R == 0;            // dB / dC summed over a wave's channels by lane swaps
     static constexpr int NP = LPR * S;
     static constexpr int NT = kCh * LPR;          // lanes per workgroup
     static constexpr int E = kT / LPR;            // steps per lane of a tile's per-element work
-    static constexpr int H = S == 2 ? 8 : 4;      // steps per reduction
+    static constexpr int H = S == 2 || SW ? 8 : 4;   // steps per reduction
+    static constexpr int NW = LPR / 4;            // waves
+    static constexpr int SR = 32 * S + 4;         // sSum stride of a step (floats)
     static constexpr int BCS = 2 * NP + 4;        // sBC row stride (floats): (B, C) pairs of a step
     static constexpr int RN = H * kRS + 2;        // sRed stride of a state (float2): its H step rows
     static constexpr int PL = LPR + 2;            // sPart stride of a step (float2)
     static constexpr int PC = H * PL + (LPR == 8 ? 8 : 0);   // sPart stride of a channel (float2)
     static constexpr int TPP = NT / (kCh * H);    // lanes that finish one (channel, step)
-    static_assert(H * NP == NT && TPP >= 1, "one dB / dC row per lane");
+    static_assert((SW || H * NP == NT) && TPP >= 1, "one dB / dC row per lane");
 };
 
+// a + its lane's counterpart in the other half (the other 16-lane row of a pair), b likewise: after the
+// swap one add leaves a's sums in the lower half (even rows) and b's in the upper (odd).
+__device__ __forceinline__ float swap_add32(float a, float b) {
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+
 template <typename T, int LPR, int S, int R>
-__global__ void __launch_bounds__(kCh * LPR) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(kCh * LPR) __attribute__((amdgpu_waves_per_eu(R == 0 && S == 2 ? 3 : 2)))
 scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck, const int64_t ck_batch,
                float *const partB, float *const partC) {
-    using Y = Layout<LPR, S>;
+    using Y = Layout<LPR, S, R>;
+    constexpr bool SW = Y::SW;
     constexpr int E = Y::E, H = Y::H, BCS = Y::BCS, NP = Y::NP, TPP = Y::TPP;
     constexpr bool AREG = S == 2 && R <= 4;   // the tile's decays stay in registers (else they spill)
     constexpr int RR = R > 0 ? R : 1;    // R = 0: no coupling, the diagonal scan
@@ -98,7 +118,9 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
     __shared__ __align__(16) float4 sX[kCh * kXS];         // [c][t]: (dt', dt'u, u, g)
     __shared__ __align__(16) float sRaw[kCh * kXS];        // [c][t]: delta + bias
     __shared__ __align__(16) float sBC[kT * BCS];          // [t][n]: (B, C)
-    __shared__ __align__(16) float2 sRed[NP * Y::RN];      // [n][t % H][c]: dB, dC terms
+    // dB, dC terms: [n][t % H][c] pairs, or (SW) [wave][t % H][lane] sums over the wave's channels.
+    __shared__ __align__(16) float2 sRed[SW ? Y::NW * H * Y::SR / 2 : NP * Y::RN];
+    float *const sSum = reinterpret_cast<float *>(sRed);
     __shared__ __align__(16) float2 sPart[kCh * Y::PC];    // [c][t % H][k]: lam B and dt' sums of a lane
     __shared__ __align__(16) float sQ[R > 0 ? kT * kCh * R : 4];   // [t][c][r]: Q h_{t-1}
 
@@ -140,10 +162,13 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
     const char *const C_p =
         reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride + g * p.C_group_stride);
     auto row_off = [&](int c, int64_t ds) { return uint32_t(c * ds) * SZ; };
-    const uint32_t fo_u = row_off(cw, p.u_d_stride), fo_d = row_off(cw, p.delta_d_stride);
-    const uint32_t fo_go = row_off(cw, p.dout_d_stride), fo_z = has_z ? row_off(cw, p.z_d_stride) : fo_go;
-    const uint32_t fo_o = has_z ? row_off(cw, p.out_d_stride) : fo_go, fo_dz = row_off(cw, p.dz_d_stride);
-    const uint32_t fo_oz = row_off(cw, p.out_z_d_stride);
+    // The lane's channel again, opaque: the row offsets below are formed once per tile from it instead of
+    // being kept in a register each.
+    auto fresh_cw = [&]() {
+        int c = cw;
+        asm volatile("" : "+v"(c));
+        return c;
+    };
 
     // The lane's rows of Q and columns of P in lane_sums order: position t holds rank t ^ ro. Every
     // rank-indexed quantity of the lane (q, P^T lam, dP, dQ) is kept in that order. At dstate <= 16
@@ -216,6 +241,10 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         constexpr bool full = decltype(full_c)::value;
         TileIn r = {};
         const int64_t t0 = j * kT;
+        const int c = fresh_cw();
+        const uint32_t fo_u = row_off(c, p.u_d_stride), fo_d = row_off(c, p.delta_d_stride);
+        const uint32_t fo_go = row_off(c, p.dout_d_stride), fo_z = has_z ? row_off(c, p.z_d_stride) : fo_go;
+        const uint32_t fo_o = has_z ? row_off(c, p.out_d_stride) : fo_go;
         const int last = last_step(t0);
         const int64_t so = t0 * SZ;
 #pragma unroll
@@ -247,6 +276,8 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         const int64_t t0 = j * kT;
         const int last = last_step(t0);
         const int64_t so = t0 * SZ;
+        const int c = fresh_cw();
+        const uint32_t fo_dz = row_off(c, p.dz_d_stride), fo_oz = row_off(c, p.out_z_d_stride);
 #pragma unroll
         for (int i = 0; i < E; ++i) {
             const bool ev = es + i <= last;
@@ -448,7 +479,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                 }
                 const float4 x = x2[t & 1];
                 const float *const Bv = B2[t & 1], *const Cv = C2[t & 1];
-                float lam[S], sv[RR], q[RR];
+                float lam[S], sv[RR], q[RR], tb[S], tc[S];
 #pragma unroll
                 for (int s = 0; s < S; ++s) lam[s] = __builtin_fmaf(Cv[s], x.w, carry[s]);
                 // P^T lam over the channel's states, rank t ^ ro at position t (as Pr, Qr, dP, dQ),
@@ -487,7 +518,24 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                         c = __builtin_fmaf(Qr[r][s], sv[r], c);
                     }
                     carry[s] = c;
-                    sRed[(k * S + s) * Y::RN + ti * kRS + cw] = make_float2(lam[s] * x.y, x.w * hs[t][s]);
+                    if constexpr (SW) {
+                        tb[s] = lam[s] * x.y;
+                        tc[s] = x.w * hs[t][s];
+                    } else {
+                        sRed[(k * S + s) * Y::RN + ti * kRS + cw] = make_float2(lam[s] * x.y, x.w * hs[t][s]);
+                    }
+                }
+                if constexpr (SW) {
+                    // Sums over the wave's 64 / LPR channels (lane / LPR): the swap of lane halves adds
+                    // dB in the lower and dC in the upper one, the swap of 16-lane rows then state 2 i in
+                    // the even and 2 i + 1 in the odd rows; with 8 lanes per channel a row holds two.
+#pragma unroll
+                    for (int i = 0; i < S; i += 2) {
+                        const float a = swap_add32(tb[i], tc[i]), b2 = swap_add32(tb[i + 1], tc[i + 1]);
+                        float v = swap_add16(a, b2);
+                        if constexpr (LPR == 8) v = dpp_add<0x128>(v);      // row_ror:8
+                        sSum[((tid >> 6) * H + ti) * Y::SR + 32 * i + (tid & 63)] = v;
+                    }
                 }
                 sPart[cw * Y::PC + ti * Y::PL + k] = make_float2(pgb, pdd);
                 if constexpr (t % 2 == 0) __builtin_amdgcn_sched_barrier(0);
@@ -501,7 +549,18 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                 for (int r = 0; r < R; ++r) asm volatile("" : "+v"(dP[s][r]), "+v"(dQ[r][s]));
             }
             __syncthreads();
-            {   // dB / dC of one (step, state) over the block's 16 channels, added pairwise in a fixed order.
+            if constexpr (SW) {   // dB / dC of S (step, state)s: the waves' sums added in order.
+#pragma unroll
+                for (int i = 0; i < S; ++i) {
+                    const int e = tid + Y::NT * i, rt = e % H, q = e / H, tz = q / NP, n = q % NP;
+                    const int at = 32 * ((n % S) & ~1) + (tz * 2 + (n & 1)) * 16 + n / S;
+                    float acc = sSum[rt * Y::SR + at];
+#pragma unroll
+                    for (int w = 1; w < Y::NW; ++w) acc += sSum[(w * H + rt) * Y::SR + at];
+                    if (tg + rt <= last && n < N)
+                        (tz == 0 ? pB : pC)[uint32_t(n) * uint32_t(Lp) + uint32_t(t0) + uint32_t(tg + rt)] = acc;
+                }
+            } else {   // dB / dC of one (step, state) over the block's 16 channels, added pairwise in a fixed order.
                 const float4 *rv = reinterpret_cast<const float4 *>(&sRed[rd_n * Y::RN + rd_t * kRS]);
                 float vb[kCh / 2], vc[kCh / 2];
 #pragma unroll
@@ -594,7 +653,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         // One dP / dQ shared by every channel: the block's 16 channels are summed in LDS first, so
         // that each element takes one atomic per block, not one per lane.
         float *const sum = reinterpret_cast<float *>(sRed);           // [dP | dQ][n][r][c]
-        static_assert(2 * NP * R * kCh <= 2 * NP * Y::RN, "the shared-P/Q sums fit sRed");
+        static_assert(SW || 2 * NP * R * kCh <= 2 * NP * Y::RN, "the shared-P/Q sums fit sRed");
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < S; ++s) {

@@ -127,6 +127,18 @@ def test_bwd_state_split(N, L, G, dtype, slots, monkeypatch):
         torch.testing.assert_close(a, b, rtol=tol, atol=tol * 0.1 * scale, msg=lambda m: f"{n}: {m}")
 
 
+@pytest.mark.parametrize("N", [1, 8, 16, 20, 32, 48, 64])
+@pytest.mark.parametrize("batch,dim,L,G", [(2, 48, 1, 1), (2, 64, 15, 2), (1, 32, 33, 1), (16, 256, 24, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_bwd_lanes_kernel(N, batch, dim, L, G, dtype):
+    """Diagonal backwards on the lane-swap reduction of scan_bwd_lanes: lengths that leave a partial
+    tile (odd ones at dstate 16 and its multiples, too), padded states, and the 256 workgroups from
+    which dstate 32 to 64 take it at any length; against the exact gradients."""
+    _say(f"bwd lanes N={N} batch={batch} dim={dim} L={L} G={G} {dtype}")
+    case = _case(880 + N + L, batch, dim, L, N, dtype, bkind="4d", G=G)
+    _vs_exact(case, _dout(881, (batch, dim, L), dtype), dtype, f"N{N} L{L}")
+
+
 @pytest.mark.parametrize("flags", [dict(with_z=False), dict(with_D=False), dict(with_bias=False),
                                    dict(softplus=False), dict(bkind="4d", G=2), dict(bkind="4d", G=4),
                                    dict(bkind="const")])
