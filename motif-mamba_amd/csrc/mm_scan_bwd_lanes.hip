@@ -31,12 +31,14 @@
 //     (lam B, dt') and (dB, dC) pairs -- one 8-byte access where two 4-byte ones, and DPP
 //     butterflies for the sums, took more instructions -- and every lane then finishes one (channel,
 //     step) and one (step, state) of them. The row strides of both keep writes and 16-byte reads at
-//     the LDS's full rate (the dstate 64 layout's dB / dC writes excepted: two-way conflicts).
-//     Without a coupling (rank 0) the dB / dC terms are instead summed over the wave's channels in
-//     registers, by swaps of lane halves and of 16-lane rows that reduce two states of both tensors at
-//     once, and only the waves' sums go through LDS: a third less LDS (23 KB at dstate 16) and no 16-term
-//     sum per row, so three waves per SIMD (8 x 1,536 channels, L 1,024, bf16: 1.63 -> 1.14 ms at dstate
-//     64, 8 x 1,024: 0.43 -> 0.36 ms at dstate 32). With P, Q, dP and dQ the registers lack the room.
+//     the LDS's full rate.
+//     Without a coupling (rank 0), and at rank 2 above dstate 16, the dB / dC terms are instead summed
+//     over the wave's channels in registers, by swaps of lane halves and of 16-lane rows that reduce two
+//     states of both tensors at once, and only the waves' sums go through LDS: a third less LDS (23 KB at
+//     dstate 16) and no 16-term sum per row, so three waves per SIMD at rank 0 (8 x 1,536 channels, L
+//     1,024, bf16: 1.63 -> 1.14 ms at dstate 64, 8 x 1,024: 0.43 -> 0.36 ms at dstate 32; training steps
+//     at rank 2, 4 x 4,096, L 1,024: 1.52 -> 1.33 ms at dstate 32, fp32 3.00 -> 2.38 ms at 64). With 8
+//     lanes per channel and a coupling it loses 1% (a third swap stage, two waves per SIMD either way).
 //   * Activations and B / C move one element at a time (uniform row bases, fixed 32-bit
 //     lane offsets), loaded one tile ahead: any length and row alignment, at
 //     about one load per step and lane group.
@@ -45,14 +47,14 @@
 //   * The states at every 16-step tile start come from the forward (its tile_states, dstate <= 16)
 //     or from a first pass that recomputes the forward into the caller's workspace.
 //
-// LDS: 40 KB (dstate 16, rank 2), 70 KB (32), 65 KB (64): four, two and two workgroups per CU, each
-// two waves per SIMD; 208 registers at dstate 16, rank 2. About 90 VALU instructions per wave-step of
+// LDS at rank 2: 40 KB (dstate 16), 39 KB (32), 51 KB (64): two waves per SIMD each; 208 registers at
+// dstate 16. About 90 VALU instructions per wave-step of
 // 8 channels x 16 states.
 //
 // Measured (rank 2, per-channel P/Q), training step of forward and backward: batch 4, 4,096 channels,
 // L 2,048, dstate 16, fp16: 1.55 -> 1.27 ms (backward 1.19 -> 0.93) against a kernel with the tile's
 // states in LDS, DPP butterflies for the du / ddelta sums and 124 VALU per wave-step; batch 8, 1,024
-// channels, L 1,024, dstate 32, bf16: 4.39 -> 0.85 ms against one lane per state.
+// channels, L 1,024, dstate 32, bf16: 4.39 -> 0.78 ms against one lane per state.
 //
 // Compiled once per input type (mm_scan_bwd_lanes_{f16,bf16}.hip include this file).
 #include <hip/hip_runtime.h>
@@ -78,7 +80,7 @@ constexpr int kRS = kCh + 2;     // sRed row stride (float2)
 
 template <int LPR, int S, int R>
 struct Layout {
-    static constexpr bool SW = R == 0;            // dB / dC summed over a wave's channels by lane swaps
+    static constexpr bool SW = R == 0 || (R == 2 && LPR == 16);   // dB / dC summed over a wave's channels by lane swaps
     static constexpr int NP = LPR * S;
     static constexpr int NT = kCh * LPR;          // lanes per workgroup
     static constexpr int E = kT / LPR;            // steps per lane of a tile's per-element work
@@ -653,7 +655,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         // One dP / dQ shared by every channel: the block's 16 channels are summed in LDS first, so
         // that each element takes one atomic per block, not one per lane.
         float *const sum = reinterpret_cast<float *>(sRed);           // [dP | dQ][n][r][c]
-        static_assert(SW || 2 * NP * R * kCh <= 2 * NP * Y::RN, "the shared-P/Q sums fit sRed");
+        static_assert(2 * NP * R * kCh <= (SW ? Y::NW * H * Y::SR : 2 * NP * Y::RN), "the shared-P/Q sums fit sRed");
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < S; ++s) {

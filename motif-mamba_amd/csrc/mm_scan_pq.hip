@@ -1065,7 +1065,7 @@ bool diag_pq_enabled() {
 
 bool diag_via_pq_fwd(const mm_scan_fwd_params &p) {
     // The tiled P/Q kernel then writes the chunk states in the diagonal form (DX), and the tile
-    // states below dstate 16 (states past dstate stay 0), which the zero-pair backward reads.
+    // states below dstate 16 (states past dstate stay 0), which the backward reads.
     if (p.P || p.dstate == 16 || p.dstate > 64 || (p.tile_states && p.dstate > 16) || !diag_pq_enabled())
         return false;
     return pq::tiled_shape(p).LPR != 0;
