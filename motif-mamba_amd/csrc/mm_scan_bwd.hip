@@ -1031,7 +1031,10 @@ SegPlan seg_plan(const mm_scan_bwd_params &p) {
     if (slots <= 0 || units == 0) return whole;
     const int64_t tail = units % slots;
     if (tail == 0) return whole;
-    int64_t n_seg = std::min<int64_t>({slots / tail, 8, n_tiles / 4});
+    // Up to 32 segments of at least 64 steps: few rows are walked in a chain of launches whose length is a
+    // segment's (bf16, against at most 8: 64 channels, L 4,096: 134 -> 67 us; 512, L 4,096: 142 -> 94 us;
+    // 1,024, L 16,384: 566 -> 432 us; 64 segments: 80, 93 and 432 us).
+    int64_t n_seg = std::min<int64_t>({slots / tail, 32, n_tiles / 4});
     if (n_seg < 2) return whole;
     const int64_t seg_tiles = (n_tiles + n_seg - 1) / n_seg;
     n_seg = (n_tiles + seg_tiles - 1) / seg_tiles;   // every segment holds at least one tile

@@ -672,3 +672,13 @@ def test_training_step_graph_replay_matches_eager():
             # in whatever order they finish.
             tol = 1e-5 if i in atomic else 0.0
             torch.testing.assert_close(a, b, rtol=tol, atol=tol, msg=lambda m: f"replay {rep}, output {i}: {m}")
+
+
+@pytest.mark.parametrize("dim,L", [(16, 2080), (32, 1026), (48, 2050)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_bwd_many_segments(dim, L, dtype):
+    """Few rows at dstate 16: up to 32 segments per row, the last one short; against the exact
+    gradients."""
+    _say(f"bwd many segments dim={dim} L={L} {dtype}")
+    case = _case(890 + dim, 1, dim, L, 16, dtype, bkind="4d", G=1)
+    _vs_exact(case, _dout(891, (1, dim, L), dtype), dtype, f"segments {dim}x{L}")
