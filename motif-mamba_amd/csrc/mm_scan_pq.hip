@@ -619,60 +619,79 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
         nn[s] = on[s] ? n0 + s : N - 1;
     }
 
-    T uv[U], dv[U], zv[U], bv[U][S], cv[U][S];
-    const int64_t ou = d * p.u_d_stride, od = d * p.delta_d_stride, oz = d * p.z_d_stride;
+    // Every load is issued before the first is waited for: no branch around one (without z, u is read in its
+    // place), and B and C stay raw words until they are used.
+    T uv[U], dv[U], zv[U];
+    RawVec<T, S> bv[U], cv[U];
+    const T *const up = reinterpret_cast<const T *>(p.u) + d * p.u_d_stride;
+    const T *const dp = reinterpret_cast<const T *>(p.delta) + d * p.delta_d_stride;
+    const T *const zp = p.z ? reinterpret_cast<const T *>(p.z) + d * p.z_d_stride : up;
+    const int64_t zb = p.z ? p.z_batch_stride : p.u_batch_stride;
     const int64_t b0 = int64_t(blockIdx.y) * U;
 #pragma unroll
     for (int i = 0; i < U; ++i) {
         const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
-        uv[i] = (reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride)[ou];
-        dv[i] = (reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride)[od];
-        if (p.z) zv[i] = (reinterpret_cast<const T *>(p.z) + b * p.z_batch_stride)[oz];
+        uv[i] = up[b * p.u_batch_stride];
+        dv[i] = dp[b * p.delta_batch_stride];
+        zv[i] = zp[b * zb];
     }
-    struct alignas(S * sizeof(T)) Four {
-        T v[S];
-    };
+    const T *const Bp = reinterpret_cast<const T *>(p.B) + g * p.B_group_stride;
+    const T *const Cp = reinterpret_cast<const T *>(p.C) + g * p.C_group_stride;
     if (bc_vec) {                          // consecutive, aligned states (uniform); no padded state in a lane
-        const int64_t ob = g * p.B_group_stride + (n0 < N ? n0 : 0), oc = g * p.C_group_stride + (n0 < N ? n0 : 0);
+        const int n = n0 < N ? n0 : 0;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
-            const Four fb = *reinterpret_cast<const Four *>(reinterpret_cast<const T *>(p.B) + b * p.B_batch_stride + ob);
-            const Four fc = *reinterpret_cast<const Four *>(reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride + oc);
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                bv[i][s] = fb.v[s];
-                cv[i][s] = fc.v[s];
-            }
+            bv[i] = load_raw<T, S>(Bp + b * p.B_batch_stride + n);
+            cv[i] = load_raw<T, S>(Cp + b * p.C_batch_stride + n);
         }
     } else {
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const int64_t ob = g * p.B_group_stride + nn[s] * p.B_dstate_stride;
-            const int64_t oc = g * p.C_group_stride + nn[s] * p.C_dstate_stride;
+        for (int i = 0; i < U; ++i) {
+            const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
+            bv[i] = cv[i] = {};
 #pragma unroll
-            for (int i = 0; i < U; ++i) {
-                const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
-                bv[i][s] = (reinterpret_cast<const T *>(p.B) + b * p.B_batch_stride)[ob];
-                cv[i][s] = (reinterpret_cast<const T *>(p.C) + b * p.C_batch_stride)[oc];
+            for (int s = 0; s < S; ++s) {
+                set_raw<T, S>(bv[i], s, load_elem<T>(reinterpret_cast<const char *>(Bp + b * p.B_batch_stride + nn[s] * p.B_dstate_stride), 0));
+                set_raw<T, S>(cv[i], s, load_elem<T>(reinterpret_cast<const char *>(Cp + b * p.C_batch_stride + nn[s] * p.C_dstate_stride), 0));
             }
         }
     }
+    // Then A, D, the bias and two ranks of Q and P at a time (clamped states: in bounds).
     float A2[S], coup[S] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < S; ++s) A2[s] = on[s] ? p.A[d * p.A_d_stride + nn[s] * p.A_dstate_stride] * kLog2e : 0.f;
-    for (int r = 0; r < int(p.pq_rank); ++r) {
-        float q = 0.f;
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-            q = __builtin_fmaf(on[s] ? p.Q[d * p.Q_d_stride + r * p.Q_r_stride + nn[s] * p.Q_dstate_stride] : 0.f, 0.f, q);
-        q = group_sum<LPR>(q);
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-            coup[s] = __builtin_fmaf(on[s] ? p.P[d * p.P_d_stride + nn[s] * p.P_dstate_stride + r * p.P_r_stride] : 0.f, q, coup[s]);
-    }
+    for (int s = 0; s < S; ++s) A2[s] = p.A[d * p.A_d_stride + nn[s] * p.A_dstate_stride];
     const float Dv = p.D ? p.D[d] : 0.f;
     const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+    const int rank = int(p.pq_rank);
+    float Qv[2][S], Pv[2][S];
+    auto load_pq = [&](int r0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int r = r0 + j < rank ? r0 + j : r0;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                Qv[j][s] = p.Q[d * p.Q_d_stride + r * p.Q_r_stride + nn[s] * p.Q_dstate_stride];
+                Pv[j][s] = p.P[d * p.P_d_stride + nn[s] * p.P_dstate_stride + r * p.P_r_stride];
+            }
+        }
+    };
+    load_pq(0);
+    for (int r0 = 0; r0 < rank; r0 += 2) {
+        if (r0 > 0) load_pq(r0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool has = r0 + j < rank;   // else zeros (a branch would take the loads behind it)
+            float q = 0.f;
+#pragma unroll
+            for (int s = 0; s < S; ++s) q = __builtin_fmaf(has && on[s] ? Qv[j][s] : 0.f, 0.f, q);
+            q = group_sum<LPR>(q);
+#pragma unroll
+            for (int s = 0; s < S; ++s) coup[s] = __builtin_fmaf(has && on[s] ? Pv[j][s] : 0.f, q, coup[s]);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) A2[s] = on[s] ? A2[s] * kLog2e : 0.f;
     const bool ls_vec = N % S == 0 && reinterpret_cast<uintptr_t>(p.last_state) % 16 == 0;
 
 #pragma unroll
@@ -683,12 +702,14 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
         if (p.delta_softplus) dt = softplus_fast(dt);
         const float uu = to_f32(uv[i]);
         const float du = dt * uu;
-        float h[S], y = 0.f;
+        float h[S], y = 0.f, Bv[S], Cv[S];
+        unpack_raw<T, S>(bv[i], Bv);
+        unpack_raw<T, S>(cv[i], Cv);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const float w = __builtin_fmaf(dt, coup[s], du * (on[s] ? to_f32(bv[i][s]) : 0.f));
+            const float w = __builtin_fmaf(dt, coup[s], du * (on[s] ? Bv[s] : 0.f));
             h[s] = __builtin_fmaf(decay_exp2(dt, A2[s]), 0.f, w);
-            y = __builtin_fmaf(h[s], on[s] ? to_f32(cv[i][s]) : 0.f, y);
+            y = __builtin_fmaf(h[s], on[s] ? Cv[s] : 0.f, y);
         }
         y = group_sum<LPR>(y);
         if (row && k == 0) {

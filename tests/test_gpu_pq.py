@@ -398,3 +398,14 @@ def test_pq_lanes_kernel_edges(N, R, L, batch, dim, bkind):
     _say(f"pq lanes N={N} R={R} L={L} batch={batch} dim={dim} {bkind}")
     case = _pq_case(900 + N + L, batch=batch, dim=dim, L=L, N=N, R=R, dtype=torch.float32, bkind=bkind)
     _vs_oracle(case, torch.float32, "lanes")
+
+
+@pytest.mark.parametrize("N,R", [(6, 3), (16, 5), (32, 4), (64, 8)])
+@pytest.mark.parametrize("with_z", [True, False], ids=["z", "noz"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
+def test_pq_step_ranks(N, R, with_z, dtype):
+    """The one-step kernel past the two ranks it holds at once, odd ranks, with B and C element by
+    element (dstate 6), without z."""
+    _say(f"pq step N={N} R={R} z={with_z} {dtype}")
+    case = _pq_case(960 + N + R, batch=5, dim=72, L=1, N=N, R=R, dtype=dtype, bkind="3d", with_z=with_z)
+    _vs_oracle(case, dtype, "step ranks")
