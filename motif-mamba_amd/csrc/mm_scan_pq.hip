@@ -594,21 +594,25 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
 // kernels' result for non-finite P, Q and decays. LPR lanes share a (batch, channel) row, four states
 // each, and serve U batch rows with one load of A, P and Q, every row's loads issued before the
 // first is used. The call moves little more than the final states, which leave as 16-byte stores of
-// consecutive lanes (one lane per row wrote each 64-byte state row in 4-byte pieces). 64 x 4,096
-// channels, dstate 16, rank 2, fp16 (20 MB): 47.5 us with one lane per row, 16.8 us here
-// (the kernel alone; 25 us when every lane also loaded its P and Q element by element for one row).
+// consecutive lanes (one lane per row wrote each 64-byte state row in 4-byte pieces). No load stands behind
+// a branch or a wait for another, addresses are a uniform base and a 32-bit lane offset, and contiguous
+// rows of A, P and Q come as vectors. Bound by the state writes beyond some 16 batch rows. 64 x 4,096
+// channels, dstate 16, rank 2, fp16 (20 MB): 45.4 us per call with one lane per row, 14.1 us here (15.7
+// with a wait per row, per rank and for B and C); 256 rows: 42 us.
 // ------------------------------------------------------------------------------------------------
 constexpr int kLanesBlock = 256;
+constexpr int kStepBC = 1, kStepAPQ = 2;   // four consecutive states per lane: of B and C, of A, P (rank 2) and Q
 
 template <typename T, int LPR, int U>
 __global__ void __launch_bounds__(kLanesBlock)
-scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t bc_vec) {
-    constexpr int S = 4;
+scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t vec) {
+    constexpr int S = 4, CPB = kLanesBlock / LPR;   // channels per block
+    constexpr uint32_t SZ = sizeof(T);
     const int k = threadIdx.x % LPR;       // states 4 k .. 4 k + 3
-    const int64_t d_raw = int64_t(blockIdx.x) * (kLanesBlock / LPR) + threadIdx.x / LPR;
-    const bool active = d_raw < p.dim;
-    const int64_t d = active ? d_raw : p.dim - 1;  // clamped for loads; stores are predicated
-    const int64_t g = d / ratio;
+    const int64_t d0 = int64_t(blockIdx.x) * CPB;
+    const int64_t left = p.dim - d0;
+    const bool active = int(threadIdx.x / LPR) < left;
+    const int dl = active ? int(threadIdx.x / LPR) : int(left) - 1;   // clamped for loads; stores are predicated
     const int N = int(p.dstate);
     const int n0 = S * k;
     int nn[S];
@@ -620,49 +624,64 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
     }
 
     // Every load is issued before the first is waited for: no branch around one (without z, u is read in its
-    // place), and B and C stay raw words until they are used.
-    T uv[U], dv[U], zv[U];
+    // place), and B and C stay raw words until they are used. Addresses are a uniform base (the batch row's
+    // or the block's first channel's) and a 32-bit lane offset, which the host has checked to fit.
+    auto base = [&](const void *t, int64_t ds) { return reinterpret_cast<const char *>(t) + d0 * ds * int64_t(SZ); };
+    const void *const zsrc = p.z ? p.z : p.u;
+    const int64_t zb = p.z ? p.z_batch_stride : p.u_batch_stride, zd = p.z ? p.z_d_stride : p.u_d_stride;
+    const char *const up = base(p.u, p.u_d_stride), *const dp = base(p.delta, p.delta_d_stride), *const zp = base(zsrc, zd);
+    const uint32_t ou = uint32_t(dl) * uint32_t(p.u_d_stride) * SZ, od = uint32_t(dl) * uint32_t(p.delta_d_stride) * SZ;
+    const uint32_t oz = uint32_t(dl) * uint32_t(zd) * SZ;
+    uint32_t uv[U], dv[U], zv[U];
     RawVec<T, S> bv[U], cv[U];
-    const T *const up = reinterpret_cast<const T *>(p.u) + d * p.u_d_stride;
-    const T *const dp = reinterpret_cast<const T *>(p.delta) + d * p.delta_d_stride;
-    const T *const zp = p.z ? reinterpret_cast<const T *>(p.z) + d * p.z_d_stride : up;
-    const int64_t zb = p.z ? p.z_batch_stride : p.u_batch_stride;
     const int64_t b0 = int64_t(blockIdx.y) * U;
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-        const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
-        uv[i] = up[b * p.u_batch_stride];
-        dv[i] = dp[b * p.delta_batch_stride];
-        zv[i] = zp[b * zb];
+        const int64_t b = (b0 + i < p.batch ? b0 + i : p.batch - 1) * int64_t(SZ);
+        uv[i] = load_elem<T>(up + b * p.u_batch_stride, ou);
+        dv[i] = load_elem<T>(dp + b * p.delta_batch_stride, od);
+        zv[i] = load_elem<T>(zp + b * zb, oz);
     }
-    const T *const Bp = reinterpret_cast<const T *>(p.B) + g * p.B_group_stride;
-    const T *const Cp = reinterpret_cast<const T *>(p.C) + g * p.C_group_stride;
-    if (bc_vec) {                          // consecutive, aligned states (uniform); no padded state in a lane
-        const int n = n0 < N ? n0 : 0;
+    // The channel's group: one for the whole block unless its channels straddle groups.
+    const int64_t g0 = p.n_groups == 1 ? 0 : d0 / ratio;
+    const uint32_t gl = p.n_groups == 1 ? 0u : uint32_t(d0 - g0 * ratio + dl) / uint32_t(ratio);
+    const char *const Bp = reinterpret_cast<const char *>(p.B) + g0 * p.B_group_stride * int64_t(SZ);
+    const char *const Cp = reinterpret_cast<const char *>(p.C) + g0 * p.C_group_stride * int64_t(SZ);
+    const uint32_t oB = gl * uint32_t(p.B_group_stride) * SZ, oC = gl * uint32_t(p.C_group_stride) * SZ;
+    if (vec & kStepBC) {                   // consecutive states (uniform); no padded state in a lane
+        const uint32_t n = uint32_t(n0 < N ? n0 : 0) * SZ;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-            const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
-            bv[i] = load_raw<T, S>(Bp + b * p.B_batch_stride + n);
-            cv[i] = load_raw<T, S>(Cp + b * p.C_batch_stride + n);
+            const int64_t b = (b0 + i < p.batch ? b0 + i : p.batch - 1) * int64_t(SZ);
+            bv[i] = load_any<T, S>(Bp + b * p.B_batch_stride, oB + n);
+            cv[i] = load_any<T, S>(Cp + b * p.C_batch_stride, oC + n);
         }
     } else {
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-            const int64_t b = b0 + i < p.batch ? b0 + i : p.batch - 1;
+            const int64_t b = (b0 + i < p.batch ? b0 + i : p.batch - 1) * int64_t(SZ);
             bv[i] = cv[i] = {};
 #pragma unroll
             for (int s = 0; s < S; ++s) {
-                set_raw<T, S>(bv[i], s, load_elem<T>(reinterpret_cast<const char *>(Bp + b * p.B_batch_stride + nn[s] * p.B_dstate_stride), 0));
-                set_raw<T, S>(cv[i], s, load_elem<T>(reinterpret_cast<const char *>(Cp + b * p.C_batch_stride + nn[s] * p.C_dstate_stride), 0));
+                set_raw<T, S>(bv[i], s, load_elem<T>(Bp + b * p.B_batch_stride, oB + uint32_t(nn[s]) * uint32_t(p.B_dstate_stride) * SZ));
+                set_raw<T, S>(cv[i], s, load_elem<T>(Cp + b * p.C_batch_stride, oC + uint32_t(nn[s]) * uint32_t(p.C_dstate_stride) * SZ));
             }
         }
     }
     // Then A, D, the bias and two ranks of Q and P at a time (clamped states: in bounds).
+    auto f32 = [&](const float *t, uint32_t off) { return __uint_as_float(load_elem<float>(reinterpret_cast<const char *>(t), off)); };
+    const float *const Ap = p.A + d0 * p.A_d_stride, *const Qp = p.Q + d0 * p.Q_d_stride, *const Pp = p.P + d0 * p.P_d_stride;
+    const uint32_t oA = 4 * uint32_t(dl) * uint32_t(p.A_d_stride), oQ = 4 * uint32_t(dl) * uint32_t(p.Q_d_stride);
+    const uint32_t oP = 4 * uint32_t(dl) * uint32_t(p.P_d_stride);
     float A2[S], coup[S] = {0.f, 0.f, 0.f, 0.f};
+    uint32_t onQ[S], onP[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) A2[s] = p.A[d * p.A_d_stride + nn[s] * p.A_dstate_stride];
-    const float Dv = p.D ? p.D[d] : 0.f;
-    const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+    for (int s = 0; s < S; ++s) {
+        onQ[s] = oQ + 4 * uint32_t(nn[s]) * uint32_t(p.Q_dstate_stride);
+        onP[s] = oP + 4 * uint32_t(nn[s]) * uint32_t(p.P_dstate_stride);
+    }
+    const float Dv = p.D ? f32(p.D + d0, 4 * uint32_t(dl)) : 0.f;
+    const float bias = p.delta_bias ? f32(p.delta_bias + d0, 4 * uint32_t(dl)) : 0.f;
     const int rank = int(p.pq_rank);
     float Qv[2][S], Pv[2][S];
     auto load_pq = [&](int r0) {
@@ -671,12 +690,35 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
             const int r = r0 + j < rank ? r0 + j : r0;
 #pragma unroll
             for (int s = 0; s < S; ++s) {
-                Qv[j][s] = p.Q[d * p.Q_d_stride + r * p.Q_r_stride + nn[s] * p.Q_dstate_stride];
-                Pv[j][s] = p.P[d * p.P_d_stride + nn[s] * p.P_dstate_stride + r * p.P_r_stride];
+                Qv[j][s] = f32(Qp + r * p.Q_r_stride, onQ[s]);
+                Pv[j][s] = f32(Pp + r * p.P_r_stride, onP[s]);
             }
         }
     };
-    load_pq(0);
+    // One vector per lane and row instead of four loads that each touch every line of the rows.
+    if (vec & kStepAPQ) {
+        const uint32_t n = 4 * uint32_t(n0 < N ? n0 : 0);
+        auto four = [&](const float *t, uint32_t off, float *o) {
+            const RawVec<float, S> v = load_any<float, S>(reinterpret_cast<const char *>(t), off);
+#pragma unroll
+            for (int s = 0; s < S; ++s) o[s] = __uint_as_float(v.w[s]);
+        };
+        four(Ap, oA + n, A2);
+        four(Qp, oQ + n, Qv[0]);
+        four(Qp + p.Q_r_stride, oQ + n, Qv[1]);
+        float p8[2 * S];
+        four(Pp, oP + 2 * n, p8);
+        four(Pp + S, oP + 2 * n, p8 + S);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            Pv[0][s] = p8[2 * s];
+            Pv[1][s] = p8[2 * s + 1];
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < S; ++s) A2[s] = f32(Ap, oA + 4 * uint32_t(nn[s]) * uint32_t(p.A_dstate_stride));
+        load_pq(0);
+    }
     for (int r0 = 0; r0 < rank; r0 += 2) {
         if (r0 > 0) load_pq(r0);
 #pragma unroll
@@ -693,14 +735,16 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
 #pragma unroll
     for (int s = 0; s < S; ++s) A2[s] = on[s] ? A2[s] * kLog2e : 0.f;
     const bool ls_vec = N % S == 0 && reinterpret_cast<uintptr_t>(p.last_state) % 16 == 0;
+    const bool write_y = active && k == 0;
+    const uint32_t oo = uint32_t(dl) * uint32_t(p.out_d_stride) * SZ, ooz = uint32_t(dl) * uint32_t(p.out_z_d_stride) * SZ;
 
 #pragma unroll
     for (int i = 0; i < U; ++i) {
         const int64_t b = b0 + i;
-        const bool row = active && b < p.batch;
-        float dt = to_f32(dv[i]) + bias;
+        if (b >= p.batch) break;           // uniform
+        float dt = elem_f32<T>(dv[i]) + bias;
         if (p.delta_softplus) dt = softplus_fast(dt);
-        const float uu = to_f32(uv[i]);
+        const float uu = elem_f32<T>(uv[i]);
         const float du = dt * uu;
         float h[S], y = 0.f, Bv[S], Cv[S];
         unpack_raw<T, S>(bv[i], Bv);
@@ -712,14 +756,17 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
             y = __builtin_fmaf(h[s], on[s] ? Cv[s] : 0.f, y);
         }
         y = group_sum<LPR>(y);
-        if (row && k == 0) {
-            const float o = p.D ? __builtin_fmaf(Dv, uu, y) : y;
-            if (p.out) (reinterpret_cast<T *>(p.out) + b * p.out_batch_stride)[d * p.out_d_stride] = from_f32<T>(o);
+        const float o = p.D ? __builtin_fmaf(Dv, uu, y) : y;
+        if (write_y) {
+            const int64_t bz = b * int64_t(SZ);
+            if (p.out)
+                store_elem<T>(reinterpret_cast<char *>(p.out) + d0 * p.out_d_stride * int64_t(SZ) + bz * p.out_batch_stride, oo, o);
             if (p.out_z)
-                (reinterpret_cast<T *>(p.out_z) + b * p.out_z_batch_stride)[d * p.out_z_d_stride] = from_f32<T>(o * silu_fast(to_f32(zv[i])));
+                store_elem<T>(reinterpret_cast<char *>(p.out_z) + d0 * p.out_z_d_stride * int64_t(SZ) + bz * p.out_z_batch_stride, ooz,
+                              o * silu_fast(elem_f32<T>(zv[i])));
         }
-        if (row && p.last_state) {
-            float *ls = p.last_state + (b * p.dim + d) * N + n0;
+        if (active && p.last_state) {
+            float *ls = p.last_state + (b * p.dim + d0) * N + (dl * N + n0);
             if (ls_vec) {
                 if (n0 < N) *reinterpret_cast<float4 *>(ls) = make_float4(h[0], h[1], h[2], h[3]);
             } else {
@@ -1016,23 +1063,35 @@ int launch_tiled_s(const mm_scan_fwd_params &p, hipStream_t s) {
     return fwd_vector_ok(&p) ? launch_tiled_v<T, S, LPR, true>(p, s) : launch_tiled_v<T, S, LPR, false>(p, s);
 }
 
+// The step kernel's 32-bit lane offsets from a block's first channel (up to 63 channels behind it, in up
+// to as many groups) must fit.
+static bool step_offsets_ok(const mm_scan_fwd_params &p) {
+    const int64_t eb = p.itype == MM_FLOAT32 ? 4 : 2, n = p.dstate - 1, lim = int64_t(1) << 32;
+    auto fits = [&](int64_t ds, int64_t ns, int64_t bytes) { return ds >= 0 && ns >= 0 && (63 * ds + n * ns + 4) * bytes < lim; };
+    return p.dim < (int64_t(1) << 31) && fits(p.u_d_stride, 0, eb) && fits(p.delta_d_stride, 0, eb) &&
+           fits(p.z ? p.z_d_stride : 0, 0, eb) && fits(p.out ? p.out_d_stride : 0, 0, eb) &&
+           fits(p.out_z ? p.out_z_d_stride : 0, 0, eb) && fits(p.B_group_stride, p.B_dstate_stride, eb) &&
+           fits(p.C_group_stride, p.C_dstate_stride, eb) && fits(p.A_d_stride, p.A_dstate_stride, 4) &&
+           fits(p.P_d_stride, p.P_dstate_stride, 4) && fits(p.Q_d_stride, p.Q_dstate_stride, 4);
+}
+
 // One-step requests with variable B and C that write no chunk or tile states take the step kernel:
 // four batch rows per workgroup where that leaves at least one workgroup per SIMD, else one.
 template <typename T, int LPR>
 int launch_lanes(const mm_scan_fwd_params &p, hipStream_t s) {
     const int64_t dblk = (p.dim + kLanesBlock / LPR - 1) / (kLanesBlock / LPR), ratio = p.dim / p.n_groups;
     const dim3 grid(unsigned(dblk), unsigned(p.batch)), block(kLanesBlock);
-    if (p.seqlen == 1 && p.is_variable_B && p.is_variable_C && !p.chunk_states && !p.tile_states) {
-        auto vec = [&](const void *ptr, int64_t bs, int64_t gs, int64_t ns) {
-            return reinterpret_cast<uintptr_t>(ptr) % (4 * sizeof(T)) == 0 && bs % 4 == 0 && gs % 4 == 0 && ns == 1;
-        };
-        const int32_t bc_vec = p.dstate % 4 == 0 && vec(p.B, p.B_batch_stride, p.B_group_stride, p.B_dstate_stride) &&
-                               vec(p.C, p.C_batch_stride, p.C_group_stride, p.C_dstate_stride);
+    if (p.seqlen == 1 && p.is_variable_B && p.is_variable_C && !p.chunk_states && !p.tile_states && step_offsets_ok(p)) {
+        int32_t vec = 0;
+        if (p.dstate % 4 == 0 && p.B_dstate_stride == 1 && p.C_dstate_stride == 1) vec |= kStepBC;
+        if (p.dstate % 4 == 0 && p.A_dstate_stride == 1 && p.Q_dstate_stride == 1 && p.pq_rank == 2 &&
+            p.P_r_stride == 1 && p.P_dstate_stride == 2)
+            vec |= kStepAPQ;
         if (dblk * ((p.batch + 3) / 4) >= device_simds())
             hipLaunchKernelGGL((scan_fwd_pq_step<T, LPR, 4>), dim3(unsigned(dblk), unsigned((p.batch + 3) / 4)), block,
-                               0, s, p, ratio, bc_vec);
+                               0, s, p, ratio, vec);
         else
-            hipLaunchKernelGGL((scan_fwd_pq_step<T, LPR, 1>), grid, block, 0, s, p, ratio, bc_vec);
+            hipLaunchKernelGGL((scan_fwd_pq_step<T, LPR, 1>), grid, block, 0, s, p, ratio, vec);
         return launch_status("scan_fwd_pq_step");
     }
     if (p.pq_rank <= 2) hipLaunchKernelGGL((scan_fwd_pq_lanes<T, LPR, 2>), grid, block, 0, s, p, ratio);
