@@ -210,7 +210,7 @@ def bench_presets(steps, warmup, torch):
     """Training steps (forward + backward through selective_scan_fn, bf16) at the Motif module's
     "small" and "base" state sizes (d_state 32 and 64, mamba_simplemotif.py:33-35), diagonal and
     with a rank-2 per-channel P/Q pair, batch 8, L 1024, 1,024 / 1,536 channels; synthetic inputs.
-    The diagonal backward runs split into groups of 16 states, the P/Q one the general kernel."""
+    Their forwards run the P/Q tiled kernel, their backwards scan_bwd_lanes."""
     from motif_mamba_amd import selective_scan_fn
     res = {}
     for kind in ("diag", "pq"):
