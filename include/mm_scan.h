@@ -219,8 +219,9 @@ typedef struct mm_scan_bwd_params {
      * torch autograd through selective_scan_full_matrix_cuda (selective_scan_interface.py:262-350,
      * its path for P/Q calls with z and for dP/dQ) both compute -- with the state adjoint running through the transposed transition matrix exp(delta' A) + delta' P Q,
      * plus dP and dQ (float32, the shapes of P and Q; overwritten: the call clears them first).
-     * Supported: variable B and C, dstate <= 16, pq_rank 1..8, dim and dim / n_groups multiples of
-     * 16, seqlen a multiple of 8; other requests return MM_ERR_UNSUPPORTED. */
+     * Any dstate <= 256, pq_rank 1..8, length, row alignment and channel count, variable or constant B
+     * and C; fastest with variable B and C, dstate <= 64 (pq_rank <= 4 above 32) and dim and
+     * dim / n_groups multiples of 16. */
     const float *P;
     const float *Q;
     int64_t pq_rank;
@@ -286,7 +287,7 @@ int mm_scan_fwd(const mm_scan_fwd_params *params, void *stream);
 
 /* Bytes of `workspace` that let mm_scan_fwd use sequence-parallel segments for this request
  * (0: the single-pass kernels are used anyway). Reads only sizes, flags and strides of `params`,
- * and the current device's compute-unit count (the segment count targets about 5 waves per SIMD):
+ * and the current device's compute-unit count (the segment count targets three to five waves per SIMD):
  * query it with the call's device current. Returns 0 for a request mm_scan_fwd would reject. No counterpart in the reference (its forward
  * allocates nothing beyond the outputs, selective_scan.cpp:383-389). */
 int64_t mm_scan_fwd_workspace_size(const mm_scan_fwd_params *params);

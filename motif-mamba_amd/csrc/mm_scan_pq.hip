@@ -12,8 +12,8 @@
 // design of this file is its own:
 //
 //   scan_fwd_pq_tiled<T, S, LPR, R>   a wave64 owns 64/LPR channels of one (batch, group), at
-//       dstate above 32 four of them in a workgroup; the LPR consecutive lanes of a channel hold S states each (S * LPR >= dstate, padded with states
-//       whose A, P, Q, B and C are zero, which stay zero). Per step each lane forms its partial
+//       dstate above 32 four of them in a workgroup; the LPR consecutive lanes of a channel hold S
+//       states each (S * LPR >= dstate, padded with states whose A, P, Q, B and C are zero, which stay zero). Per step each lane forms its partial
 //       Q h over its S states, a DPP butterfly inside the LPR lanes sums the partials (every lane
 //       ends with the same bits; where the rank is at most LPR one transposed butterfly serves all
 //       R sums, lane_sums in mm_common.h), and the lane updates its S states with
