@@ -1884,11 +1884,16 @@ static bool k2s_bytes_ok(const mm_scan_fwd_params &p) {
     return span * size < (int64_t(1) << 32);
 }
 
+// Whether the request has output rows at all. k2s, k1s and the mixed grid store theirs without asking
+// (their instances are built for out, out_z or both); a request for states alone (z and out NULL)
+// belongs to the kernels that look at the pointer: k2i, the pipelined and the row-per-lane kernel.
+static bool has_rows(const mm_scan_fwd_params &p) { return p.out || p.out_z; }
+
 // Requests of any length and row alignment that the ragged k2s takes: inference (no chunk or tile
 // states, one output), from kMinRagged steps on.
 constexpr int64_t kMinRagged = 8;
 static bool ragged_ok(const mm_scan_fwd_params &p) {
-    if (p.dstate != 16 || !p.is_variable_B || !p.is_variable_C || p.chunk_states || p.tile_states || (p.z && p.out))
+    if (!has_rows(p) || p.dstate != 16 || !p.is_variable_B || !p.is_variable_C || p.chunk_states || p.tile_states || (p.z && p.out))
         return false;
     if (p.dim % tiled::kCh != 0 || (p.dim / p.n_groups) % tiled::kCh != 0) return false;
     // Rows start on whole elements.
@@ -1907,10 +1912,10 @@ static bool ragged_route(const mm_scan_fwd_params &p) {
 }
 
 // Whether a segmented request runs on k2s: every 32-step pair whole, byte offsets in range, and
-// neither a request that writes both out and out_z nor fp32 with chunk states (the pipelined
-// kernel's segments serve those; MM_SCAN_KERNEL=k2 selects them always).
+// neither a request that writes both out and out_z, nor one without either, nor fp32 with chunk
+// states (the pipelined kernel's segments serve those; MM_SCAN_KERNEL=k2 selects them always).
 static bool k2s_segments_ok(const mm_scan_fwd_params &p) {
-    return p.seqlen % (2 * tiled::kT1) == 0 && tiled_variant() != 20 && !(p.z && p.out) &&
+    return has_rows(p) && p.seqlen % (2 * tiled::kT1) == 0 && tiled_variant() != 20 && !(p.z && p.out) &&
            !(p.itype == MM_FLOAT32 && p.chunk_states) && k2s_bytes_ok(p);
 }
 
@@ -2004,12 +2009,12 @@ static bool mix_plan(const mm_scan_fwd_params &p, int32_t &n_double, int32_t &n_
 }
 
 // The two-states-per-lane kernels: k2s (symmetric element work, or the balanced mixed grid) when L
-// is a multiple of 32 and the byte offsets fit, else k2i for 16-bit inputs (MM_SCAN_KERNEL=k2i
-// selects k2i always, for comparison) and the pipelined kernel for fp32.
+// is a multiple of 32, the byte offsets fit and there are output rows to write, else k2i for 16-bit
+// inputs (MM_SCAN_KERNEL=k2i selects k2i always, for comparison) and the pipelined kernel for fp32.
 template <typename T>
 static int launch_k2x(const mm_scan_fwd_params &p, hipStream_t stream) {
     static const bool nofull = getenv("MM_SCAN_NOFULL") != nullptr;
-    const bool whole_pairs = p.seqlen % (2 * tiled::kT1) == 0 && !nofull && k2s_bytes_ok(p);
+    const bool whole_pairs = has_rows(p) && p.seqlen % (2 * tiled::kT1) == 0 && !nofull && k2s_bytes_ok(p);
     int32_t n_double = 0, n_single = 0;
     if constexpr (sizeof(T) == 4) {
         // fp32: k2s for the inference requests it compiles for (no chunk or tile states), the

@@ -680,3 +680,36 @@ def test_segment_counts(n_seg, L, monkeypatch):
     case = _case(190 + n_seg, 2, 32, L, 16, torch.bfloat16, bkind="4d", G=1)
     out, last = _run(case)
     _rows_vs_f64(case, out, last, f"n_seg={n_seg} L={L}")
+
+
+@pytest.mark.parametrize("dim,L", [(32, 33), (32, 37), (32, 64), (32, 1024), (32, 1100), (32, 8192), (0, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("off", [0, 1], ids=["aligned", "odd-rows"])
+def test_states_without_output_rows(dim, L, dtype, off):
+    """mm_scan_fwd with z and out both NULL: only last_state (and, asked for, chunk_states) is wanted.
+    Ragged and whole pairs, with the queried workspace (segments) and without, and (dim 0 here: three
+    16-channel groups per compute unit) the shape of the mixed grid; the states against the float64
+    restatement."""
+    lib = capi.load()
+    batch, dim = (2, dim) if dim else (1, 3 * _cus() * 16)
+    _say(f"states alone dim={dim} L={L} {dtype} off={off}")
+    case = _case(210, batch, dim, L, 16, dtype, bkind="4d", G=1, with_z=False, with_D=False)
+    g = _to(case, DEV)
+    wide = lambda t: torch.cat([t.new_zeros(*t.shape[:-1], off), t], dim=-1)[..., off:]   # noqa: E731
+    u, delta = wide(g["u"]), wide(g["delta"])
+    exp = cscan.scan_all_rows(**case)[1]
+    for with_chunks in (False, True):
+        for with_ws in (False, True):
+            last = torch.full((batch, dim, 16), float("nan"), device=DEV)
+            chunks = torch.full((batch, dim, (L + 2047) // 2048, 32), float("nan"), device=DEV) if with_chunks else None
+            p = capi.scan_fwd_params(u, delta, g["A"], g["B"], g["C"], delta_bias=g["delta_bias"],
+                                     delta_softplus=True, last_state=last, chunk_states=chunks)
+            ws = torch.empty(max(16, lib.mm_scan_fwd_workspace_size(ctypes.byref(p))), dtype=torch.uint8, device=DEV)
+            if with_ws:
+                p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+            assert lib.mm_scan_fwd(ctypes.byref(p), capi.stream_handle()) == 0, lib.mm_last_error()
+            torch.cuda.synchronize()
+            rtol, atol = fixtures.tolerances(dtype)
+            np.testing.assert_allclose(last.cpu().double().numpy(), exp, rtol=rtol, atol=atol)
+            if with_chunks:
+                assert torch.equal(chunks[:, :, -1, 1::2], last)
