@@ -1076,12 +1076,14 @@ static bool step_offsets_ok(const mm_scan_fwd_params &p) {
 }
 
 // One-step requests with variable B and C that write no chunk or tile states take the step kernel:
-// four batch rows per workgroup where that leaves at least one workgroup per SIMD, else one.
+// four batch rows per workgroup where that leaves at least one workgroup per SIMD, else one. It reads a
+// first rank of P and Q before it looks at the rank: at rank 0, where P and Q hold no element,
+// scan_fwd_pq_lanes serves the call, whose every access stands behind r < rank.
 template <typename T, int LPR>
 int launch_lanes(const mm_scan_fwd_params &p, hipStream_t s) {
     const int64_t dblk = (p.dim + kLanesBlock / LPR - 1) / (kLanesBlock / LPR), ratio = p.dim / p.n_groups;
     const dim3 grid(unsigned(dblk), unsigned(p.batch)), block(kLanesBlock);
-    if (p.seqlen == 1 && p.is_variable_B && p.is_variable_C && !p.chunk_states && !p.tile_states && step_offsets_ok(p)) {
+    if (p.seqlen == 1 && p.pq_rank >= 1 && p.is_variable_B && p.is_variable_C && !p.chunk_states && !p.tile_states && step_offsets_ok(p)) {
         int32_t vec = 0;
         if (p.dstate % 4 == 0 && p.B_dstate_stride == 1 && p.C_dstate_stride == 1) vec |= kStepBC;
         if (p.dstate % 4 == 0 && p.A_dstate_stride == 1 && p.Q_dstate_stride == 1 && p.pq_rank == 2 &&

@@ -409,3 +409,25 @@ def test_pq_step_ranks(N, R, with_z, dtype):
     _say(f"pq step N={N} R={R} z={with_z} {dtype}")
     case = _pq_case(960 + N + R, batch=5, dim=72, L=1, N=N, R=R, dtype=dtype, bkind="3d", with_z=with_z)
     _vs_oracle(case, dtype, "step ranks")
+
+
+@pytest.mark.parametrize("N", [16, 32, 64])
+def test_pq_rank_zero_one_step_c_abi(N):
+    """mm_scan_fwd with rank 0 (no coupling), P and Q given, and one time step: P and Q hold no element,
+    so nothing of them may be read; the outputs are the diagonal scan's."""
+    _say(f"P/Q rank 0, L 1, dstate {N}")
+    lib = capi.load()
+    case = _pq_case(300 + N, batch=2, dim=48, L=1, N=N, R=1, dtype=torch.float16)
+    del case["P"], case["Q"]
+    g = _to(case, DEV)
+    out_z, last = torch.empty_like(g["u"]), torch.empty(2, 48, N, device=DEV)
+    p = capi.scan_fwd_params(g["u"], g["delta"], g["A"], g["B"].unsqueeze(1), g["C"].unsqueeze(1), g["D"], g["z"],
+                             g["delta_bias"], True, out_z=out_z, last_state=last)
+    anywhere = torch.full((1,), float("nan"), device=DEV)
+    p.P = p.Q = anywhere.data_ptr()
+    p.pq_rank = 0
+    assert lib.mm_scan_fwd(ctypes.byref(p), capi.stream_handle()) == 0, lib.mm_last_error()
+    torch.cuda.synchronize()
+    ref, ref_last = selective_scan_ref(**case, return_last_state=True)
+    _close(out_z.cpu(), ref, torch.float16, "rank 0 out_z")
+    _close(last.cpu(), ref_last, torch.float16, "rank 0 last")
