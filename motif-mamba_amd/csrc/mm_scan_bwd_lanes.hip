@@ -432,9 +432,14 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                 __builtin_amdgcn_sched_barrier(0);
             });
         }
-        // sQ is written and read by the lanes of one wave (a channel's), whose LDS accesses stay in
-        // order; the barrier is for the compiler.
-        if constexpr (R > 0) __builtin_amdgcn_wave_barrier();
+        // sQ is written by one lane of a channel and read by the others, all lanes of one wave, whose LDS
+        // accesses the hardware keeps in order. The fences keep the compiler from moving a read before
+        // the store (the wave barrier alone orders no memory); at this scope they emit no instruction.
+        if constexpr (R > 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        }
         float4 xn[2];
         float Bn[2][S], Cn[2][S], qn[2][RR];
         auto read = [&](int t) __attribute__((always_inline)) {
