@@ -232,13 +232,16 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         co[i] = uint32_t((n < N ? n : 0) * p.C_dstate_stride) * SZ;
     }
 
-    // A tile's global inputs as raw elements, loaded one tile ahead of their use. Steps past L are
-    // clamped to the row's last element (they are padding: dt' = g = 0, B = C = 0).
+    // A tile's global inputs as raw elements, loaded one tile ahead of their use. A row's last, partial
+    // tile is right-aligned: position i holds step i - sh of the tile, the sh positions before its first
+    // step (clamped to that step) are padding with dt' = u = g = 0 and B = C = 0. Padding in front only
+    // meets the tile's entry state and passes it, and the adjoint, on unchanged; behind the last step it
+    // would meet that step's own state, where 0 times an infinite state is NaN in dA, dP and dQ.
     struct TileIn {
         uint32_t d[E], u[E], go[E], z[E], o[E], b[S], c[S];
         float hck[S];
     };
-    auto last_step = [&](int64_t t0) { return int(L - 1 - t0 < kT - 1 ? L - 1 - t0 : kT - 1); };
+    auto padding = [&](int64_t t0) { return int(L - t0 < kT ? kT - (L - t0) : 0); };
     auto fetch = [&](int64_t j, auto full_c, bool with_ck) __attribute__((always_inline)) {
         constexpr bool full = decltype(full_c)::value;
         TileIn r = {};
@@ -247,11 +250,11 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
         const uint32_t fo_u = row_off(c, p.u_d_stride), fo_d = row_off(c, p.delta_d_stride);
         const uint32_t fo_go = row_off(c, p.dout_d_stride), fo_z = has_z ? row_off(c, p.z_d_stride) : fo_go;
         const uint32_t fo_o = has_z ? row_off(c, p.out_d_stride) : fo_go;
-        const int last = last_step(t0);
+        const int sh = padding(t0);
         const int64_t so = t0 * SZ;
 #pragma unroll
         for (int i = 0; i < E; ++i) {
-            const uint32_t eo = uint32_t(es + i < last ? es + i : last) * SZ;
+            const uint32_t eo = uint32_t(max(es - sh + i, 0)) * SZ;
             r.d[i] = load_elem<T>(d_p + so, fo_d + eo);
             r.u[i] = load_elem<T>(u_p + so, fo_u + eo);
             if constexpr (full) {
@@ -260,7 +263,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                 r.o[i] = load_elem<T>(o_p + so, fo_o + eo);
             }
         }
-        const uint32_t to = uint32_t(st_t < last ? st_t : last) * SZ;
+        const uint32_t to = uint32_t(max(st_t - sh, 0)) * SZ;
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             r.b[i] = load_elem<T>(B_p + so, bo[i] + to);
@@ -276,14 +279,14 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
     auto commit = [&](int64_t j, auto full_c, const TileIn &r) __attribute__((always_inline)) {
         constexpr bool full = decltype(full_c)::value;
         const int64_t t0 = j * kT;
-        const int last = last_step(t0);
+        const int sh = padding(t0);
         const int64_t so = t0 * SZ;
         const int c = fresh_cw();
         const uint32_t fo_dz = row_off(c, p.dz_d_stride), fo_oz = row_off(c, p.out_z_d_stride);
 #pragma unroll
         for (int i = 0; i < E; ++i) {
-            const bool ev = es + i <= last;
-            const float uu = elem_f32<T>(r.u[i]);
+            const bool ev = es - sh + i >= 0;
+            const float uu = ev ? elem_f32<T>(r.u[i]) : 0.f;
             float go = 0.f;
             if constexpr (full) {
                 go = elem_f32<T>(r.go[i]);
@@ -292,7 +295,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                     const float oo = elem_f32<T>(r.o[i]);
                     const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-zz * kLog2e));
                     if (ev) {
-                        const uint32_t eo = uint32_t(es + i) * SZ;
+                        const uint32_t eo = uint32_t(es - sh + i) * SZ;
                         store_elem<T>(dz_p + so, fo_dz + eo, go * oo * sg * (1.f + zz * (1.f - sg)));
                         if (has_oz) store_elem<T>(oz_p + so, fo_oz + eo, oo * zz * sg);
                     }
@@ -307,7 +310,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const int n = st_n + LPR * i;
-            const bool on = n < N && st_t <= last;
+            const bool on = n < N && st_t >= sh;
             const float bv = on ? elem_f32<T>(r.b[i]) : 0.f;
             if constexpr (full)
                 *reinterpret_cast<float2 *>(&sBC[st_t * BCS + 2 * n]) = make_float2(bv, on ? elem_f32<T>(r.c[i]) : 0.f);
@@ -373,7 +376,7 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
     TileIn in = fetch(n_tiles - 1, kFull, true);
     for (int64_t j = n_tiles - 1; j >= 0; --j) {
         const int64_t t0 = j * kT;
-        const int last = last_step(t0);
+        const int sh = padding(t0);
         float hck[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) hck[s] = in.hck[s];
@@ -564,8 +567,8 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                     float acc = sSum[rt * Y::SR + at];
 #pragma unroll
                     for (int w = 1; w < Y::NW; ++w) acc += sSum[(w * H + rt) * Y::SR + at];
-                    if (tg + rt <= last && n < N)
-                        (tz == 0 ? pB : pC)[uint32_t(n) * uint32_t(Lp) + uint32_t(t0) + uint32_t(tg + rt)] = acc;
+                    if (tg + rt - sh >= 0 && n < N)
+                        (tz == 0 ? pB : pC)[uint32_t(n) * uint32_t(Lp) + uint32_t(t0) + uint32_t(tg + rt - sh)] = acc;
                 }
             } else {   // dB / dC of one (step, state) over the block's 16 channels, added pairwise in a fixed order.
                 const float4 *rv = reinterpret_cast<const float4 *>(&sRed[rd_n * Y::RN + rd_t * kRS]);
@@ -584,8 +587,8 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                         vc[i] += vc[i + w];
                     }
                 }
-                if (tg + rd_t <= last && rd_n < N) {
-                    const uint32_t o = rd_off + uint32_t(t0) + uint32_t(tg + rd_t);
+                if (rd_t - sh + tg >= 0 && rd_n < N) {
+                    const uint32_t o = rd_off + uint32_t(t0) + uint32_t(rd_t - sh + tg);
                     pB[o] = vb[0];
                     pC[o] = vc[0];
                 }
@@ -611,9 +614,9 @@ scan_bwd_lanes(const mm_scan_bwd_params p, const int64_t ratio, float *const ck,
                 }
                 const float4 x = sX[fc * kXS + t];
                 const float raw = sRaw[fc * kXS + t];
-                if (t <= last) {
+                if (ft - sh + tg >= 0) {
                     const int64_t so = t0 * SZ;
-                    const uint32_t to = uint32_t(t) * SZ;
+                    const uint32_t to = uint32_t(ft - sh + tg) * SZ;
                     if (fsub == 0) {
                         store_elem<T>(du_p + so, fo_du + to, __builtin_fmaf(Dv, x.w, x.x * gb));
                         dD_acc = __builtin_fmaf(x.w, x.z, dD_acc);

@@ -496,6 +496,39 @@ def test_pq_bwd_lanes_edges(N, R, L, per_dim, dtype, monkeypatch):
         _check(gr, exact["d" + n], dtype, f"lanes d{n}")
 
 
+@pytest.mark.parametrize("N,R", [(8, 0), (16, 0), (16, 2), (16, 8), (32, 0), (32, 2), (64, 0), (64, 4)])
+@pytest.mark.parametrize("L", [15, 33])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_bwd_lanes_infinite_last_step(N, R, L, dtype, monkeypatch):
+    """An infinite u at a row's last step, in a tile that the row does not fill: every gradient that does
+    not hold that element (dA, dP and dQ hold the states up to the step before, du none) has the bits it
+    has with a finite one."""
+    _say(f"bwd lanes, infinite last u, N={N} R={R} L={L} {dtype}")
+    monkeypatch.setenv("MM_SCAN_PAD", "0")
+    from motif_mamba_amd import selective_scan_fn
+    case = _pq_case(870 + N + L, batch=1, dim=32, L=L, N=N, R=max(R, 1), dtype=dtype, with_z=False, with_D=False)
+    if R == 0:
+        del case["P"], case["Q"]
+    names = [n for n in NAMES if torch.is_tensor(case.get(n))]
+    dout = _dout(871, (1, 32, L), dtype).to(DEV)
+
+    def grads(last):
+        g = {k: (v.to(DEV) if torch.is_tensor(v) else v) for k, v in case.items()}
+        g["u"] = g["u"].clone()
+        g["u"][..., -1] = last
+        for n in names:
+            g[n].requires_grad_(True)
+        out = selective_scan_fn(**g)
+        return dict(zip(names, torch.autograd.grad(out, [g[n] for n in names], dout)))
+
+    a, b = grads(1.0), grads(float("inf"))
+    for n in names:
+        if n == "delta_bias":                 # the sum of ddelta, the last step's among them
+            continue
+        cut = slice(None, L - 1) if n in ("delta", "B", "C") else slice(None)
+        assert torch.isfinite(a[n]).all() and torch.equal(a[n][..., cut], b[n][..., cut]), n
+
+
 def test_pq_bwd_batch_rows_in_several_launches():
     """Slabs of five batch rows exceed the 4 GiB one launch takes: four rows, then one. Each row's own
     gradients equal those of the row alone bit for bit; the parameters' are their sum (float32
