@@ -1937,17 +1937,20 @@ int64_t device_simds() {
 }
 
 // Sequence segments for shapes whose (batch, 16-channel) groups give fewer than one wave per SIMD
-// (two waves per group), past 1,024 steps: shorter rows stay whole, so that inference keeps the bits of
-// the training forward there, which is not cut (the carry reassociates the sums of three segments and
-// more; 512 channels, L 1,024: 46 us whole, 19 us in 16 segments).
-// Two plans: as many segments of at least 64 steps as give three waves per SIMD, or of at least 512
-// steps as give five, whichever needs fewer rounds of waves per step of a segment. bf16,
+// (two waves per group). Up to 1,504 steps (47 tile pairs) rows are cut in two at most, from 1,024 on:
+// two segments keep the bits of the whole row (the second starts from the first's end state as it is), and
+// so inference those of the training forward, which is not cut; the carry of three and more reassociates
+// sums. (1 x 5,120 channels, L 1,024, bf16: 68 us in two, 70 whole. More segments would be faster: 512, L
+// 1,024: 19 us in 16, 46 whole or in two; 2,560, L 1,280: 37 in 13, 70 in two.)
+// Past that, two plans: as many segments of at least 64 steps as give three waves per SIMD, or of at least
+// 512 steps as give five, whichever needs fewer rounds of waves per step of a segment. bf16,
 // against at most five waves per SIMD of at least 512 steps: 512 channels, L 2,048: 47 -> 22 us; 1,536,
 // L 2,048: 68 -> 36 us; 2 x 1,536, L 1,777: 94 -> 58 us; 3 x 2,560, L 8,192: 434 -> 421 us. From 1,024
 // waves on whole rows win (2 x 5,120, L 2,048: 136 us, 153 to 163 in segments).
 // Long rows: 160 groups, L 65,536, fp32, 6, 8, 9, 10, 12, 15, 16, 19, 24 and 32 segments take 1.42,
 // 1.44, 1.31, 1.48, 1.40, 1.29, 1.24, 1.24, 1.25 and 1.25 ms. MM_SCAN_SEGMENTS=n sets the count (for
 // measurements).
+constexpr int64_t kMaxPairsInTwo = 47;
 int64_t segment_count(const mm_scan_fwd_params &p) {
     if (!ragged_route(p) && (!tiled_shape_ok(p) || !fwd_vector_ok(&p) || !pipe_offsets_ok(p) || p.tile_states)) return 1;
     const int64_t waves = 2 * p.batch * (p.dim / tiled::kCh);
@@ -1957,11 +1960,11 @@ int64_t segment_count(const mm_scan_fwd_params &p) {
         n_seg = std::min<int64_t>(std::atoll(e), n_pairs);
     } else {
         const int64_t simds = device_simds();
-        if (waves >= simds || p.seqlen <= 1024) return 1;
+        if (waves >= simds) return 1;
         const int64_t few = std::min(3 * simds / waves, n_pairs / 2);
         const int64_t many = std::min((5 * simds + waves - 1) / waves, n_pairs / 16);
         auto rounds = [&](int64_t n) { return (waves * n + simds - 1) / simds; };
-        n_seg = rounds(many) * few < rounds(few) * many ? many : few;
+        n_seg = n_pairs <= kMaxPairsInTwo || rounds(many) * few < rounds(few) * many ? many : few;
     }
     if (n_seg < 2) return 1;
     const int64_t pairs = (n_pairs + n_seg - 1) / n_seg;

@@ -713,3 +713,20 @@ def test_states_without_output_rows(dim, L, dtype, off):
             np.testing.assert_allclose(last.cpu().double().numpy(), exp, rtol=rtol, atol=atol)
             if with_chunks:
                 assert torch.equal(chunks[:, :, -1, 1::2], last)
+
+
+@pytest.mark.parametrize("L", [992, 1024, 1025, 1280, 1357, 1504])
+@pytest.mark.parametrize("dim", [64, 1024])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_inference_has_the_training_forward_bits_up_to_two_segments(L, dim, dtype):
+    """Rows that inference cuts in two at most (up to 1,504 steps) keep the bits of the training forward,
+    which is not cut: the second segment starts from the first one's end state as it is."""
+    _say(f"inference and training bits L={L} dim={dim} {dtype}")
+    from motif_mamba_amd import selective_scan_fn
+    g = _to(_case(41, 2, dim, L, 16, dtype), DEV)
+    out, last = selective_scan_fn(**g, return_last_state=True)
+    g["A"].requires_grad_(True)
+    out_train, last_train = selective_scan_fn(**g, return_last_state=True)
+    torch.cuda.synchronize()
+    assert out_train.requires_grad
+    assert torch.equal(out, out_train.detach()) and torch.equal(last, last_train.detach())
