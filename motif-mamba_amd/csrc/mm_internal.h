@@ -35,6 +35,8 @@ int64_t segment_workspace_bytes(const mm_scan_fwd_params &p, int64_t n_seg);
 // SIMDs of the current device (4 per CU; cached per device), 1024 when it cannot be queried
 // (mm_scan_tiled.hip).
 int64_t device_simds();
+// Whether a diagonal dstate-16 forward runs on the kernel for any length and row alignment.
+bool ragged_route(const mm_scan_fwd_params &p);
 
 // Forward scan with the low-rank P/Q coupling (mm_scan_pq.hip): the tiled kernel when the request
 // fits it, else the lane-per-row kernel.

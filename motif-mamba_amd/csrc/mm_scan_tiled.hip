@@ -1889,6 +1889,7 @@ static bool k2s_bytes_ok(const mm_scan_fwd_params &p) {
 // belongs to the kernels that look at the pointer: k2i, the pipelined and the row-per-lane kernel.
 static bool has_rows(const mm_scan_fwd_params &p) { return p.out || p.out_z; }
 
+#ifdef MM_TILED_COMMON
 // Requests of any length and row alignment that the ragged k2s takes: inference (no chunk or tile
 // states, one output), from kMinRagged steps on.
 constexpr int64_t kMinRagged = 8;
@@ -1902,14 +1903,19 @@ static bool ragged_ok(const mm_scan_fwd_params &p) {
         if (reinterpret_cast<uintptr_t>(t) % eb) return false;
     return p.seqlen >= kMinRagged && p.batch <= 65535 && k2s_bytes_ok(p);
 }
-// Whether the request takes it. Aligned rows keep the buffer-addressed kernels where every tile pair is
-// whole, at 8 and 16 steps (batch 64, 5,120 channels, bf16, L 8: 64 us against 88 us), and where a
-// variant is forced for measurements.
-static bool ragged_route(const mm_scan_fwd_params &p) {
+// Whether the request takes it. Aligned rows of a multiple of 8 steps keep the buffer-addressed kernels,
+// whole or in segments: 16-bit ones without whole tile pairs k2i (4 x 5,120 channels, L 200, bf16: 28.7 us
+// against 31.3; 16 x 5,120, L 24: 21.1 against 24.7; in segments 2 x 1,536, L 1,544: 53.4 against 55.4), float32 ones
+// the pipelined kernel (16 x 5,120, L 24: 17.2 against 25.2; L 1,000: 430 against 440). Only long 16-bit
+// rows with five waves per SIMD are faster here (8 x 5,120, L 1,000: 217 -> 200 us, L 2,040: 437 -> 388; at
+// L 520 105 against 108; with 2.5 waves, 4 x 5,120, L 2,040: 226 against 228).
+bool ragged_route(const mm_scan_fwd_params &p) {
     if (!ragged_ok(p)) return false;
-    const bool aligned = fwd_vector_ok(&p) && tiled_shape_ok(p);
-    return !aligned || !(p.seqlen % (2 * tiled::kT1) == 0 || p.seqlen <= tiled::kT1 || tiled_variant() != 0);
+    if (!fwd_vector_ok(&p) || !tiled_shape_ok(p)) return true;
+    if (p.seqlen % (2 * tiled::kT1) == 0 || tiled_variant() != 0) return false;
+    return p.itype != MM_FLOAT32 && p.seqlen >= 768 && 2 * p.batch * (p.dim / tiled::kCh) >= 5 * device_simds();
 }
+#endif  // MM_TILED_COMMON
 
 // Whether a segmented request runs on k2s: every 32-step pair whole, byte offsets in range, and
 // neither a request that writes both out and out_z, nor one without either, nor fp32 with chunk

@@ -355,3 +355,37 @@ def test_causal_conv1d_import_paths_and_argument_errors():
                                       False, True)
     with pytest.raises(RuntimeError):       # CPU tensors are refused by the binding
         causal_conv1d.causal_conv1d_fn(x, w)
+
+
+def test_which_rows_take_the_kernel_for_any_alignment():
+    """The diagonal dstate-16 forward's route (mm::ragged_route; 1,024 SIMDs where no device is there):
+    aligned rows of a multiple of 8 steps stay on the buffer-addressed kernels, but long 16-bit ones with
+    five waves per SIMD; odd lengths and rows leave them; requests without output rows stay, too."""
+    lib = capi.load()
+    route = lib._ZN2mm12ragged_routeERK18mm_scan_fwd_params
+    route.argtypes, route.restype = [ctypes.POINTER(capi.ScanFwdParams)], ctypes.c_bool
+    f32, bf16 = 0, 2
+
+    def goes(batch, dim, L, itype, base=4096, **kw):
+        p = capi.ScanFwdParams()
+        p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.itype = batch, dim, L, 16, 1, itype
+        p.is_variable_B = p.is_variable_C = 1
+        p.u = p.delta = p.A = p.B = p.C = p.z = p.out_z = base
+        p.u_batch_stride = p.delta_batch_stride = p.z_batch_stride = p.out_z_batch_stride = dim * L
+        p.u_d_stride = p.delta_d_stride = p.z_d_stride = p.out_z_d_stride = L
+        p.B_batch_stride = p.C_batch_stride = p.B_group_stride = p.C_group_stride = 16 * L
+        p.B_dstate_stride = p.C_dstate_stride = L
+        for k, v in kw.items():
+            setattr(p, k, v)
+        return route(ctypes.byref(p))
+
+    for itype in (f32, bf16):
+        for L in (8, 16, 24, 40, 200, 520, 1000, 1784, 4088, 4096):
+            assert not goes(2, 1536, L, itype), (L, itype)
+        for L in (17, 33, 1777, 4095):
+            assert goes(2, 1536, L, itype), (L, itype)
+            assert not goes(2, 1536, L, itype, z=None, out_z=None, last_state=4096), (L, itype)
+        assert goes(2, 1536, 4096, itype, base=4096 + 4)         # whole pairs of unaligned rows
+        assert not goes(2, 1536, 33, itype, chunk_states=8192)   # training
+    assert goes(8, 5120, 1000, bf16) and goes(8, 5120, 776, bf16) and not goes(8, 5120, 520, bf16)
+    assert not goes(7, 5120, 1000, bf16) and not goes(8, 5120, 1024, bf16) and not goes(8, 5120, 1000, f32)
