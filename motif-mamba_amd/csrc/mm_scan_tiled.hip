@@ -1890,9 +1890,25 @@ static bool k2s_bytes_ok(const mm_scan_fwd_params &p) {
 static bool has_rows(const mm_scan_fwd_params &p) { return p.out || p.out_z; }
 
 #ifdef MM_TILED_COMMON
+// Steps from which the ragged k2s is the faster kernel for rows outside the aligned ones: it always scans a
+// whole tile pair, the row-per-lane kernel only the row's steps, one after the other. With few rows the
+// chain of steps decides (8 x 5,120 channels, L 8: 29.8 us against 15.2 in bf16, 18.6 against 14.7 in fp32),
+// with many the work (row-per-lane against ragged, us):
+//                             L 8          L 9          L 10         L 12         L 13         L 14
+//   bf16   64 x 2,048      34.0 36.1    46.9 36.2
+//          64 x 5,120      66.7 83.7    92.3 84.7
+//          256 x 5,120      242 334      327 333      348 333
+//   fp32   64 x 2,048      23.9 34.2    34.6 34.2
+//          64 x 5,120      48.3 79.7    68.4 79.8    71.4 79.9    78.7 80.0    82.6 80.0
+//          256 x 5,120      157 300      225 302      234 302      262 301      274 306      298 313
+static int64_t min_ragged(const mm_scan_fwd_params &p) {
+    const int64_t waves = 2 * p.batch * (p.dim / tiled::kCh) / device_simds();   // of the ragged kernel per SIMD
+    if (p.itype == MM_FLOAT32) return waves >= 128 ? 15 : waves >= 32 ? 13 : waves >= 16 ? 9 : 8;
+    return waves >= 128 ? 10 : waves >= 16 ? 9 : 8;
+}
+
 // Requests of any length and row alignment that the ragged k2s takes: inference (no chunk or tile
-// states, one output), from kMinRagged steps on.
-constexpr int64_t kMinRagged = 8;
+// states, one output), from min_ragged steps on.
 static bool ragged_ok(const mm_scan_fwd_params &p) {
     if (!has_rows(p) || p.dstate != 16 || !p.is_variable_B || !p.is_variable_C || p.chunk_states || p.tile_states || (p.z && p.out))
         return false;
@@ -1901,7 +1917,7 @@ static bool ragged_ok(const mm_scan_fwd_params &p) {
     const uintptr_t eb = p.itype == MM_FLOAT32 ? 4 : 2;
     for (const void *t : {p.u, p.delta, p.z, p.B, p.C, static_cast<const void *>(p.out), static_cast<const void *>(p.out_z)})
         if (reinterpret_cast<uintptr_t>(t) % eb) return false;
-    return p.seqlen >= kMinRagged && p.batch <= 65535 && k2s_bytes_ok(p);
+    return p.seqlen >= min_ragged(p) && p.batch <= 65535 && k2s_bytes_ok(p);
 }
 // Whether the request takes it. Aligned rows of a multiple of 8 steps keep the buffer-addressed kernels,
 // whole or in segments: 16-bit ones without whole tile pairs k2i (4 x 5,120 channels, L 200, bf16: 28.7 us

@@ -389,3 +389,7 @@ def test_which_rows_take_the_kernel_for_any_alignment():
         assert not goes(2, 1536, 33, itype, chunk_states=8192)   # training
     assert goes(8, 5120, 1000, bf16) and goes(8, 5120, 776, bf16) and not goes(8, 5120, 520, bf16)
     assert not goes(7, 5120, 1000, bf16) and not goes(8, 5120, 1024, bf16) and not goes(8, 5120, 1000, f32)
+    # Few steps of many rows stay on the row-per-lane kernel (odd rows at 8 steps).
+    for itype, batch, first in ((bf16, 8, 8), (bf16, 64, 9), (bf16, 256, 10), (f32, 8, 8), (f32, 64, 13), (f32, 256, 15)):
+        for L in range(8, 16):
+            assert goes(batch, 5120, L, itype, base=4096 + 4) == (L >= first), (itype, batch, L)
