@@ -235,6 +235,12 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     // Loads at or past the end of a row are redirected into the row's last elements (always in
     // bounds: L is a multiple of 8, or element by element); the steps they feed are padding with
     // dt' = 0 (and, where a lane's steps may be part padding, u = 0).
+    // PEEL: without VEC the partial tile comes after the loop, in code of its own, where a lane holds four
+    // states and stages B and C alone: with it in the loop the rank-2 instance spilled 69 registers in fp32 and 20
+    // at 16 bits (18 and none so; rank 8, fp16: 108 and 80), 64 x 4,096 channels, L 21, rank 8, dstate 16, fp16: 338 ->
+    // 196 us; 24 x 4,096, L 255, rank 8, fp32: 631 -> 580. The other layouts have the registers, and the partial
+    // tile's inputs in flight a tile ahead are worth more (2 x 1,536, L 777, dstate 64, fp32: 81 against 87 us).
+    constexpr bool PEEL = !VEC && S == 4 && W == 1;
     const int64_t lastE = L - E;
     const char *const ub = reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.u) + b * p.u_batch_stride + dw * p.u_d_stride);
     const char *const db = reinterpret_cast<const char *>(reinterpret_cast<const T *>(p.delta) + b * p.delta_batch_stride + dw * p.delta_d_stride);
@@ -249,6 +255,16 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     struct Elems {
         RawVec<T, E> u, d, z;
     };
+    auto load_part = [&](int64_t t, Elems &e) {   // of a partial tile, element by element
+        e = {};
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const uint32_t eo = uint32_t(t + es + i < L ? t + es + i : L - 1) * SZ;
+            set_raw<T, E>(e.u, i, load_elem<T>(ub, fo_u + eo));
+            set_raw<T, E>(e.d, i, load_elem<T>(db, fo_d + eo));
+            if (zp) set_raw<T, E>(e.z, i, load_elem<T>(zb, fo_z + eo));
+        }
+    };
     auto load_elems = [&](int64_t t, Elems &e) {
         if constexpr (!VEC) {
             if (t + kT <= L) {             // uniform: a whole tile
@@ -258,15 +274,8 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
                 e.d = load_any<T, E>(db + so, fo_d + eo);
                 if (zp) e.z = load_any<T, E>(zb + so, fo_z + eo);
                 else e.z = {};
-            } else {
-                e = {};
-#pragma unroll
-                for (int i = 0; i < E; ++i) {
-                    const uint32_t eo = uint32_t(t + es + i < L ? t + es + i : L - 1) * SZ;
-                    set_raw<T, E>(e.u, i, load_elem<T>(ub, fo_u + eo));
-                    set_raw<T, E>(e.d, i, load_elem<T>(db, fo_d + eo));
-                    if (zp) set_raw<T, E>(e.z, i, load_elem<T>(zb, fo_z + eo));
-                }
+            } else if (!PEEL && t < L) {
+                load_part(t, e);
             }
             return;
         }
@@ -309,7 +318,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
                 r.c[i] = buffer_load_rawn<T, 8>(rs_C, fo_C[i] + o, 0);
                 if (st >= L) r.b[i] = r.c[i] = {};
             }
-        }                                  // without VEC stage_bc loads that tile
+        }                                  // without VEC stage_part loads that tile
         if (padded) {
 #pragma unroll
             for (int i = 0; i < NU; ++i)
@@ -317,26 +326,29 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         }
     };
     // Tile rows [step][B states | C states] as float32 (zeros for padded states and past L).
+    auto stage_part = [&](int64_t t0) {    // the partial tile, element by element
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+            uint32_t vb[8], vc[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int64_t st = t0 + 8 * u_q + e;
+                const uint32_t o = uint32_t(st < L ? st : L - 1) * SZ;
+                vb[e] = load_elem<T>(Bb, fo_B[i] + o);
+                vc[e] = load_elem<T>(Cb, fo_C[i] + o);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool on = u_on[i] && t0 + 8 * u_q + e < L;
+                sBC[u_lds + 16 * W * i + e * BCS] = on ? elem_f32<T>(vb[e]) : 0.f;
+                sBC[u_lds + 16 * W * i + e * BCS + NP] = on ? elem_f32<T>(vc[e]) : 0.f;
+            }
+        }
+    };
     auto stage_bc = [&](const BCs &r, int64_t t0) {
-        if constexpr (!VEC) {
-            if (t0 + kT > L) {             // uniform: the partial tile, element by element
-#pragma unroll
-                for (int i = 0; i < NU; ++i) {
-                    uint32_t vb[8], vc[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int64_t st = t0 + 8 * u_q + e;
-                        const uint32_t o = uint32_t(st < L ? st : L - 1) * SZ;
-                        vb[e] = load_elem<T>(Bb, fo_B[i] + o);
-                        vc[e] = load_elem<T>(Cb, fo_C[i] + o);
-                    }
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const bool on = u_on[i] && t0 + 8 * u_q + e < L;
-                        sBC[u_lds + 16 * W * i + e * BCS] = on ? elem_f32<T>(vb[e]) : 0.f;
-                        sBC[u_lds + 16 * W * i + e * BCS + NP] = on ? elem_f32<T>(vc[e]) : 0.f;
-                    }
-                }
+        if constexpr (!VEC && !PEEL) {
+            if (t0 + kT > L) {             // uniform
+                stage_part(t0);
                 return;
             }
         }
@@ -366,26 +378,33 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
     };
     Elems e0, e1;
     BCs b0, b1;
-    load_elems(0, e0);
-    if (D == 2) load_elems(kT, e1);
-    load_bc(0, b0);
-    stage_bc(b0, 0);
-    pin(e0, b0);
-    if (D == 2) load_bc(kT, b1);
+    const int64_t Lt = PEEL ? L - L % kT : L;   // end of the loop's tiles
+    if (!PEEL || Lt > 0) {
+        load_elems(0, e0);
+        if (D == 2) load_elems(kT, e1);
+        load_bc(0, b0);
+        stage_bc(b0, 0);
+        pin(e0, b0);
+        if (D == 2) load_bc(kT, b1);
+    }
 
     // Tile t0: its elements in ec, its B/C (already staged) in bc, the next tile's B/C in bn (the
-    // same entry as bc when D = 1: loaded at the top of the tile, staged at its end).
-    auto tile = [&](const int64_t t0, Elems &ec, BCs &bc, Elems &en, BCs &bn) __attribute__((always_inline)) {
+    // same entry as bc when D = 1: loaded at the top of the tile, staged at its end). TAIL: PEEL's partial
+    // tile, which nothing follows.
+    auto tile = [&](auto tail_c, const int64_t t0, Elems &ec, BCs &bc, Elems &en, BCs &bn) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail_c)::value, WHOLE = PEEL && !TAIL;
         const int64_t t1 = t0 + kT;
         // This lane's elements exist: all or none of them where L is a multiple of E.
-        auto ev = [&](int i) { return VEC ? t0 + es < L : t0 + es + i < L; };
+        auto ev = [&](int i) { return VEC ? t0 + es < L : WHOLE || t0 + es + i < L; };
         float uu[E], dd[E], zz[E];
         unpack_raw<T, E>(ec.u, uu);
         unpack_raw<T, E>(ec.d, dd);
         unpack_raw<T, E>(ec.z, zz);
         // Prefetch D tiles ahead into the entries just consumed (clamped addresses: in bounds).
-        load_elems(t0 + D * kT, ec);
-        load_bc(t0 + D * kT, bc);
+        if constexpr (!TAIL) {
+            load_elems(t0 + D * kT, ec);
+            load_bc(t0 + D * kT, bc);
+        }
 
         // Prologue: dt' and dt' u of (channel, steps es .. es + E - 1).
         float dtp[E], dup[E];
@@ -508,12 +527,12 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
 #pragma unroll
         for (int t = 0; t < kT; t += 4)
             *reinterpret_cast<float4 *>(&sY[(cw * LPR + k) * kPad + t]) = make_float4(yp[t], yp[t + 1], yp[t + 2], yp[t + 3]);
-        if (t1 < L) stage_bc(bn, t1);
+        if (!TAIL && t1 < Lt) stage_bc(bn, t1);
         // The next tile's inputs are taken as read here, where they have long arrived: at their first use
         // (or, B and C, at the next loads into their registers) the wait for them would be one for the
         // stores below or for the loads just issued as well (2,048 channels, L 30,001, dstate 64, rows of
         // any alignment: 3.7 -> 2.8 ms).
-        pin(en, bn);
+        if constexpr (!TAIL) pin(en, bn);
         __syncthreads();
 
         // Epilogue: y of (channel, steps es .. es + E - 1) = the LPR partials, added in lane order.
@@ -537,7 +556,7 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
             auto put = [&](auto rs, char *base, uint32_t off) __attribute__((always_inline)) {
                 if constexpr (VEC) {
                     buffer_store_vecn<T, E>(rs, off, uint32_t(t0) * SZ, o);
-                } else if (t1 <= L) {      // uniform
+                } else if (WHOLE || (!TAIL && t1 <= L)) {   // uniform
                     store_any<T, E>(base + t0 * SZ, off, o);
                 } else {
 #pragma unroll
@@ -569,13 +588,21 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         }
         __syncthreads();                   // sY reads done before the next prologue overwrites sX
     };
+    constexpr std::false_type kLoop{};
     if constexpr (D == 2) {
-        for (int64_t t0 = 0; t0 < L; t0 += 2 * kT) {
-            tile(t0, e0, b0, e1, b1);
-            if (t0 + kT < L) tile(t0 + kT, e1, b1, e0, b0);
+        for (int64_t t0 = 0; t0 < Lt; t0 += 2 * kT) {
+            tile(kLoop, t0, e0, b0, e1, b1);
+            if (t0 + kT < Lt) tile(kLoop, t0 + kT, e1, b1, e0, b0);
         }
     } else {
-        for (int64_t t0 = 0; t0 < L; t0 += kT) tile(t0, e0, b0, e0, b0);
+        for (int64_t t0 = 0; t0 < Lt; t0 += kT) tile(kLoop, t0, e0, b0, e0, b0);
+    }
+    if constexpr (PEEL) {
+        if (Lt < L) {                      // uniform; the loop's last barrier stands behind its reads of sBC
+            load_part(Lt, e0);
+            stage_part(Lt);
+            tile(std::true_type{}, Lt, e0, b0, e0, b0);
+        }
     }
     if (active && p.last_state) {
         float *ls = p.last_state + (b * p.dim + d) * N;

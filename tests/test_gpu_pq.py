@@ -411,6 +411,31 @@ def test_pq_step_ranks(N, R, with_z, dtype):
     _vs_oracle(case, dtype, "step ranks")
 
 
+@pytest.mark.parametrize("L", [9, 31, 32, 33, 63, 65, 97])
+@pytest.mark.parametrize("N,lpr,R", [(16, 4, 2), (13, 4, 8), (32, 8, 2), (27, 8, 4), (16, 8, 2), (16, 16, 2), (64, 16, 3)])
+@pytest.mark.parametrize("train", [False, True], ids=["inference", "training"])
+def test_pq_unaligned_rows_every_layout(L, N, lpr, R, train):
+    """Rows off 16-byte alignment in each layout, with no, one and several whole tiles before a partial
+    one (which the four-states-per-lane layouts run after their loop) and without a partial one; the
+    training forward writes the chunk states and (dstate <= 16) the tile states from it, too."""
+    _say(f"pq unaligned rows L={L} N={N} lpr={lpr} R={R} train={train}")
+    from motif_mamba_amd import selective_scan_fn
+    case = _pq_case(700 + N + L, batch=2, dim=40, L=L, N=N, R=R, dtype=torch.float32, bkind="4d", G=1)
+    g = _to(case, DEV)
+    for k in ("u", "z", "B"):                  # rows of an (L + 3)-wide tensor, from column 1
+        w = torch.zeros(*g[k].shape[:-1], L + 3, device=DEV)
+        w[..., 1:L + 1] = g[k]
+        g[k] = w[..., 1:L + 1]
+    if train:
+        g["P"].requires_grad_(True)
+    with _lpr(lpr):
+        out, last = selective_scan_fn(**g, return_last_state=True)
+        torch.cuda.synchronize()
+    ref, ref_last = selective_scan_pq_ref(**case, return_last_state=True)
+    _close(out.detach().cpu(), ref, torch.float32, "out")
+    _close(last.detach().cpu(), ref_last, torch.float32, "last")
+
+
 @pytest.mark.parametrize("N", [16, 32, 64])
 def test_pq_rank_zero_one_step_c_abi(N):
     """mm_scan_fwd with rank 0 (no coupling), P and Q given, and one time step: P and Q hold no element,
