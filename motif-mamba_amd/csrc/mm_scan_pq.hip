@@ -1170,6 +1170,28 @@ bool diag_pq_enabled() {
     const char *e = getenv("MM_DIAG_VIA_PQ");
     return !(e && e[0] == '0');
 }
+
+// Inference rows shorter than half a tile, odd or unaligned, of many channels: the tiled kernel stages a tile's
+// worth of B and C element by element whatever the length, the row-per-lane kernel's work grows with length
+// times dstate (us, row-per-lane against tiled):
+//              16 x 4,096 channels                        64 x 4,096 channels
+//              L 8          L 9          L 13             L 8          L 9          L 13         L 15
+//   fp16  4    14.2 22.2    19.8 22.4    22.6 22.9        28.3 80.1    39.4 81.5    50.7 84.1    56.3 84.1
+//         8    19.0 22.2    26.4 22.4                     39.3 80.5    54.2 81.8    68.8 84.4    76.7 84.2
+//         12   24.1 22.2    33.5 22.5                     49.0 80.6    67.8 82.1    86.1 84.7    96.2 84.7
+//         32                                              116  101
+//   fp32  4    11.5 20.4    16.7 20.5    19.8 21.2        23.7 73.5    33.6 74.0    43.0 75.6    48.4 75.8
+//         8    13.8 20.5    20.4 20.6    23.8 21.3        30.0 73.7    42.4 74.1    52.3 75.9    59.5 75.8
+//         12   16.6 20.6    24.6 20.8    28.8 21.5        34.6 74.3    49.5 74.7    61.1 75.8    68.5 75.9
+//         32                                              78.6 102     110  104
+// and with fewer rows the tiled kernel wins (8 x 4,096, dstate 8, L 9, fp16: 25.9 against 12.6).
+bool short_rows(const mm_scan_fwd_params &p) {
+    if (p.seqlen >= 16 || p.chunk_states || p.tile_states || fwd_vector_ok(&p)) return false;
+    const int64_t waves = p.batch * p.dim / 8 / device_simds(), work = p.seqlen * p.dstate;   // eight-lane waves per SIMD
+    const bool f32 = p.itype == MM_FLOAT32;
+    if (waves >= 32) return work <= (!f32 ? 150 : p.seqlen == 8 ? 256 : 200);
+    return waves >= 8 && work <= (f32 ? 100 : p.seqlen == 8 ? 64 : 44);
+}
 }  // namespace
 
 bool diag_via_pq_fwd(const mm_scan_fwd_params &p) {
@@ -1177,6 +1199,7 @@ bool diag_via_pq_fwd(const mm_scan_fwd_params &p) {
     // states below dstate 16 (states past dstate stay 0), which the backward reads.
     if (p.P || p.dstate == 16 || p.dstate > 64 || (p.tile_states && p.dstate > 16) || !diag_pq_enabled())
         return false;
+    if (short_rows(p)) return false;
     return pq::tiled_shape(p).LPR != 0;
 }
 

@@ -393,3 +393,32 @@ def test_which_rows_take_the_kernel_for_any_alignment():
     for itype, batch, first in ((bf16, 8, 8), (bf16, 64, 9), (bf16, 256, 10), (f32, 8, 8), (f32, 64, 13), (f32, 256, 15)):
         for L in range(8, 16):
             assert goes(batch, 5120, L, itype, base=4096 + 4) == (L >= first), (itype, batch, L)
+
+
+def test_which_short_rows_leave_the_pq_kernels():
+    """The diagonal forward at dstate != 16 (mm::diag_via_pq_fwd): odd or unaligned inference rows shorter
+    than 16 steps of many channels run on the row-per-lane kernel, up to a length times dstate."""
+    lib = capi.load()
+    route = lib._ZN2mm15diag_via_pq_fwdERK18mm_scan_fwd_params
+    route.argtypes, route.restype = [ctypes.POINTER(capi.ScanFwdParams)], ctypes.c_bool
+
+    def goes(batch, L, N, itype, base=4096 + 4, **kw):
+        p = capi.ScanFwdParams()
+        p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.itype = batch, 4096, L, N, 1, itype
+        p.is_variable_B = p.is_variable_C = 1
+        p.u = p.delta = p.A = p.B = p.C = p.z = p.out_z = base
+        p.u_batch_stride = p.delta_batch_stride = p.z_batch_stride = p.out_z_batch_stride = 4096 * L
+        p.u_d_stride = p.delta_d_stride = p.z_d_stride = p.out_z_d_stride = L
+        p.B_batch_stride = p.C_batch_stride = p.B_group_stride = p.C_group_stride = N * L
+        p.B_dstate_stride = p.C_dstate_stride = L
+        for k, v in kw.items():
+            setattr(p, k, v)
+        return route(ctypes.byref(p))
+
+    f32, f16 = 0, 1
+    for itype, batch, N, last in ((f16, 64, 4, 15), (f16, 64, 12, 12), (f16, 64, 32, 7), (f32, 64, 8, 15), (f32, 64, 32, 8),
+                                  (f16, 16, 4, 11), (f16, 16, 8, 8), (f32, 16, 8, 12), (f32, 8, 4, 7), (f16, 1, 1, 7)):
+        for L in range(8, 20):
+            assert goes(batch, L, N, itype) == (L > last), (itype, batch, N, L)
+    assert goes(64, 8, 4, f16, base=4096) and goes(64, 9, 4, f16, chunk_states=8192)
+    assert not goes(64, 7, 4, f16) and not goes(64, 32, 16, f16)
