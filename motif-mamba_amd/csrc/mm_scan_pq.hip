@@ -1058,13 +1058,16 @@ static TiledShape tiled_shape(const mm_scan_fwd_params &p) {
     // 4 lanes); past that the 4-lane layout's half as many waves win (0.45 against 0.55 ms at 3).
     // Without a coupling the lanes of a channel only meet in y: bf16, L 2048, 2,048 channels x batch 4
     // (1,024 waves of 8 lanes): 0.183 against 0.199 ms at dstate 32, equal at dstate 8; with 1,536 such
-    // waves 0.150 against 0.138 and 0.134 against 0.094 ms, and 4 lanes stay behind 8 (dstate 8, 2,560
-    // waves of 8: 0.296 against 0.244 ms).
+    // waves 0.150 against 0.138 and 0.134 against 0.094 ms. 4 lanes stay behind 8 up to 2.5 waves of 8 per
+    // SIMD (dstate 8, L 2048: 0.296 against 0.244 ms) and win past that on aligned rows (4 against 8 lanes,
+    // dstate 4 and 12 alike, us: 3 per SIMD, L 512, fp16 77 90, fp32 77 84; 4: 80 106, 82 100; 5: 119 118,
+    // 129 142; 16: 303 339, 313 406; 32, L 8: 44 53, 44 66). Unaligned rows keep 8: there the partial tile costs a
+    // lane of four states more (32 per SIMD, L 63, fp32: 134 against 126).
     const int64_t simds = device_simds();
     if (nc == 1) return cands[0];
-    if (!p.P) return waves(16) <= 2 * simds ? cands[nc - 1] : (nc == 3 ? cands[1] : cands[0]);
-    if (waves(16) <= simds) return cands[nc - 1];
+    if (waves(16) <= (p.P ? 1 : 2) * simds) return cands[nc - 1];
     if (nc == 2) return cands[0];
+    if (!p.P && !fwd_vector_ok(&p)) return cands[1];
     return 2 * waves(8) <= 5 * simds ? cands[1] : cands[0];
 }
 

@@ -730,3 +730,32 @@ def test_inference_has_the_training_forward_bits_up_to_two_segments(L, dim, dtyp
     torch.cuda.synchronize()
     assert out_train.requires_grad
     assert torch.equal(out, out_train.detach()) and torch.equal(last, last_train.detach())
+
+
+@pytest.mark.parametrize("N", [1, 7, 12, 15])
+@pytest.mark.parametrize("L", [8, 40, 2080])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_four_lanes_per_channel_without_a_coupling(N, L, dtype, monkeypatch):
+    """The layout that diagonal requests of many channels at dstate below 16 take (forced here): one and
+    several tiles, a partial one, a part-filled last wave; every row's output and last state against the
+    float64 restatement, and the training forward's, with chunk and tile states, against inference."""
+    monkeypatch.setenv("MM_PQ_LPR", "4")
+    _say(f"four lanes per channel N={N} L={L} {dtype}")
+    from motif_mamba_amd import _native, selective_scan_fn
+    case = _case(230 + N + L, 2, 48, L, N, dtype, bkind="4d", G=2)
+    g = _to(case, DEV)
+    out, last = selective_scan_fn(**g, return_last_state=True)
+    _, x, out_z, ck = _native.ext().fwd(g["u"], g["delta"], g["A"], g["B"], g["C"], g["D"], g["z"], g["delta_bias"],
+                                        None, None, None, True, tile_states=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out, out_z) and torch.equal(last, x[:, :, -1, 1::2])
+    rows = [(b, d) for b in (0, 1) for d in range(48)]
+    r = cscan.scan_rows(**case, rows=rows, chunk=16)
+    rtol, atol = fixtures.tolerances(dtype)
+    exact = torch.from_numpy(r["out_z"]).reshape(2, 48, L)
+    err = (out.cpu().double() - exact).abs().amax(dim=-1)
+    assert bool((err <= atol + rtol * exact.abs().amax(dim=-1)).all())
+    states = np.concatenate([np.zeros((96, 1, N)), r["h_chunks"][:, :(L - 1) // 16]], axis=1)
+    got = ck.reshape(ck.shape[0], 96, 16).permute(1, 0, 2).cpu().double().numpy()
+    np.testing.assert_allclose(got[..., :N], states, rtol=1e-3, atol=1e-3)
+    assert not got[..., N:].any()
