@@ -531,8 +531,9 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
         // The next tile's inputs are taken as read here, where they have long arrived: at their first use
         // (or, B and C, at the next loads into their registers) the wait for them would be one for the
         // stores below or for the loads just issued as well (2,048 channels, L 30,001, dstate 64, rows of
-        // any alignment: 3.7 -> 2.8 ms).
-        if constexpr (!TAIL) pin(en, bn);
+        // any alignment: 3.7 -> 2.8 ms). Not where a lane's four states spill with rank 8 in fp32: aligned rows,
+        // dstate 32, 2 x 4,096 channels, L 2,048: 768 us with it, 756 without (16 x 4,096, L 512: 1,112 and 1,093).
+        if constexpr (!TAIL && !(VEC && S == 4 && R == 8 && SZ == 4)) pin(en, bn);
         __syncthreads();
 
         // Epilogue: y of (channel, steps es .. es + E - 1) = the LPR partials, added in lane order.
