@@ -193,14 +193,16 @@ def test_workspace_size_query():
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(bad)) == 0                      # invalid request
     assert lib.mm_scan_fwd_workspace_size(None) == 0
     odd = params(1, 2560, 65536, itype=0)
-    odd.u = 4098                         # rows not 16-byte aligned: the row-per-lane kernel, no segments
+    odd.u = 4100                         # rows not 16-byte aligned: the ragged kernel, in segments as well
+    assert lib.mm_scan_fwd_workspace_size(ctypes.byref(odd)) == seg
+    odd.u = 4098                         # not on whole elements: the row-per-lane kernel, no segments
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(odd)) == 0
 
 
 def test_tile_states_size_query(monkeypatch):
     """mm_scan_fwd_tile_states_size (sizes, flags, strides and pointer alignment only; fake pointers
     are never dereferenced): the training forward of the dstate-16 kernels, the diagonal training
-    forward below dstate 16 (the P/Q kernels with a zero coupling) and every P/Q request with
+    forward below dstate 16 (the P/Q kernels without a coupling, any length) and every P/Q request with
     dstate <= 16 write them; other requests do not."""
     lib = capi.load()
 
@@ -226,7 +228,8 @@ def test_tile_states_size_query(monkeypatch):
     assert size(params(4, 5120, 4096)) == 256 * 4 * 5120 * 16 * 4           # config 2 training forward
     assert size(params(2, 64, 200)) == 13 * 2 * 64 * 16 * 4                 # ragged last tile
     assert size(params(4, 5120, 4096, chunks=False)) == 0                  # the inference forward
-    assert size(params(2, 64, 256, N=8)) == 16 * 2 * 64 * 16 * 4           # zero-coupling P/Q kernels
+    assert size(params(2, 64, 256, N=8)) == 16 * 2 * 64 * 16 * 4           # P/Q kernels, no coupling
+    assert size(params(2, 64, 100, N=8)) == 7 * 2 * 64 * 16 * 4            # of any length
     monkeypatch.setenv("MM_DIAG_VIA_PQ", "0")
     assert size(params(2, 64, 256, N=8)) == 0                              # that route off: none
     monkeypatch.delenv("MM_DIAG_VIA_PQ")

@@ -91,11 +91,11 @@ def test_bwd_shapes(dtype, N):
 
 
 @pytest.mark.parametrize("N", [1, 4, 8, 12])
-@pytest.mark.parametrize("via_pq", ["1", "0"], ids=["zero-pair", "general"])
+@pytest.mark.parametrize("via_pq", ["1", "0"], ids=["pq-kernels", "general"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["fp32", "bf16", "fp16"])
 def test_bwd_small_dstate(N, via_pq, dtype, monkeypatch):
     """Diagonal training at dstate < 16 (variable B/C): the forward and the backward on the P/Q
-    kernels with a zero rank-1 pair (the forward's tile states handed over), or (MM_DIAG_VIA_PQ=0)
+    kernels without a coupling (the forward's tile states handed over), or (MM_DIAG_VIA_PQ=0)
     on the general kernels; against the exact gradients, 3 dtypes."""
     monkeypatch.setenv("MM_DIAG_VIA_PQ", via_pq)
     _say(f"bwd dstate {N} via_pq={via_pq} {dtype}")
@@ -148,10 +148,11 @@ def test_bwd_options(flags):
     _vs_exact(case, _dout(611, (2, 32, 100), torch.float32), torch.float32, str(flags))
 
 
-@pytest.mark.parametrize("pad", ["1", "0"], ids=["padded", "general"])
+@pytest.mark.parametrize("pad", ["1", "0"], ids=["padded", "as-is"])
 @pytest.mark.parametrize("L", [1, 7, 2049, 4100, 2056, 4096])
 def test_bwd_lengths(L, pad, monkeypatch):
-    """Odd lengths run padded (the fast kernels) or, with MM_SCAN_PAD=0, on the general kernels."""
+    """Lengths that are not multiples of 8 run padded, or, with MM_SCAN_PAD=0, as they are: the general
+    training forward and the dstate-16 backward (even lengths) or scan_bwd_lanes (odd ones)."""
     monkeypatch.setenv("MM_SCAN_PAD", pad)
     _say(f"bwd L={L} padding {pad}")
     case = _case(620 + L, 1, 16, L, 16, torch.float32)
@@ -371,9 +372,9 @@ def test_bwd_tile_states(dtype, monkeypatch):
 @pytest.mark.parametrize("N", [4, 8, 12])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_bwd_tile_states_small_dstate(N, dtype):
-    """Below dstate 16 the training forward runs on the P/Q kernels with a zero coupling and writes
+    """Below dstate 16 the training forward runs on the P/Q kernels without a coupling and writes
     the tile states too (ck[j] = the state after the first 16 j steps, states past dstate 0); the
-    zero-coupling backward reading them matches the one recomputing them to float32 rounding, and
+    backward reading them matches the one recomputing them to float32 rounding, and
     both match the exact gradients."""
     _say(f"bwd tile states dstate {N} {dtype}")
     from motif_mamba_amd import _native
@@ -517,10 +518,10 @@ def test_bwd_states_pass_balanced_grid(q, dtype):
 @pytest.mark.parametrize("L,dtype,N", [(13, torch.float32, 16), (1001, torch.bfloat16, 16), (2047, torch.float32, 16),
                                        (13, torch.float32, 8), (1001, torch.bfloat16, 4)])
 def test_bwd_padded_lengths(L, dtype, N):
-    """Training at lengths that are not multiples of 8: selective_scan_fn pads the request in front
-    with zero-u steps (forward and backward on the padded copies, gradients of the real steps
-    returned); the output, last state and every gradient against the exact ones. dstate 16 runs
-    the diagonal kernels, dstate 8 and 4 the P/Q ones with a zero pair."""
+    """Training at lengths that are not multiples of 8. At dstate 16 selective_scan_fn pads the request in
+    front with zero-u steps (forward and backward on the padded copies, gradients of the real steps
+    returned); dstate 8 and 4 run unpadded on the P/Q kernels without a coupling. The output, last
+    state and every gradient against the exact ones."""
     _say(f"bwd padded length L={L} {dtype} dstate {N}")
     from motif_mamba_amd import selective_scan_fn
     case = _case(760 + L + N, 2, 64, L, N, dtype, bkind="4d", G=2)

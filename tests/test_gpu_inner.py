@@ -129,11 +129,11 @@ def test_backward(dtype, ckpt, bc_bias):
         _check(gg[k], v, dtype, f"d{k}")
 
 
-@pytest.mark.parametrize("pad", ["1", "0"], ids=["padded", "general"])
+@pytest.mark.parametrize("pad", ["1", "0"], ids=["padded", "as-is"])
 @pytest.mark.parametrize("ckpt", [0, 1])
 def test_backward_without_biases_ragged_length(pad, ckpt, monkeypatch):
     """L = 37: the scan runs on copies padded in front with zero-u steps (forward and backward), or,
-    with MM_SCAN_PAD=0, on the general kernels."""
+    with MM_SCAN_PAD=0, as it is (the general training forward and scan_bwd_lanes)."""
     monkeypatch.setenv("MM_SCAN_PAD", pad)
     _say(f"mamba_inner bwd no biases L=37 padding {pad} checkpoint_lvl={ckpt}")
     c = _case(920, L=37, biases=False)

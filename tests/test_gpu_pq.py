@@ -164,19 +164,18 @@ def test_pq_general_large_dstate(N):
     _vs_oracle(case, torch.float32, f"N{N}")
 
 
-@pytest.mark.parametrize("pad", ["0", "1"], ids=["general", "padded"])
-def test_pq_general_odd_length_and_strided_rows(pad, monkeypatch):
-    """Odd L with misaligned u rows: the lane-per-row P/Q kernel (MM_SCAN_PAD=0), or the fast
-    kernel on the binding's front-padded copies."""
-    _say(f"pq odd L and strided u, padding {pad}")
-    monkeypatch.setenv("MM_SCAN_PAD", pad)
+@pytest.mark.parametrize("L", [7, 37], ids=["lanes", "tiled"])
+def test_pq_general_odd_length_and_strided_rows(L):
+    """Odd L with misaligned u rows: below 8 steps the kernel of four states per lane, from there on the
+    tiled one for any alignment."""
+    _say(f"pq odd L={L} and strided u")
     from motif_mamba_amd import selective_scan_fn
-    case = _pq_case(380, batch=2, dim=16, L=37, N=16, R=2, dtype=torch.bfloat16)
+    case = _pq_case(380, batch=2, dim=16, L=L, N=16, R=2, dtype=torch.bfloat16)
     g = _to(case, DEV)
-    wide = torch.zeros(2, 16, 41, dtype=torch.bfloat16, device=DEV)
-    wide[:, :, 2:39] = g["u"]
-    g["u"] = wide[:, :, 2:39]              # stride(-1) == 1, row starts not 16-byte aligned
-    assert g["u"].stride() == (16 * 41, 41, 1)
+    wide = torch.zeros(2, 16, L + 4, dtype=torch.bfloat16, device=DEV)
+    wide[:, :, 2:L + 2] = g["u"]
+    g["u"] = wide[:, :, 2:L + 2]           # stride(-1) == 1, row starts not 16-byte aligned
+    assert g["u"].stride() == (16 * (L + 4), L + 4, 1)
     out, last = selective_scan_fn(**g, return_last_state=True)
     ref, ref_last = selective_scan_pq_ref(**case, return_last_state=True)
     _close(out.cpu(), ref, torch.bfloat16, "odd L out")
@@ -184,13 +183,13 @@ def test_pq_general_odd_length_and_strided_rows(pad, monkeypatch):
 
 
 @pytest.mark.parametrize("L,R", [(1, 2), (4, 2), (5, 2), (1001, 2), (2047, 4)])
-def test_pq_padded_length(L, R):
-    """P/Q inference at lengths that are not multiples of 8: from 5 steps on the fast kernel on
-    front-padded copies (zero u keeps the coupled state at zero through the padding), below the
-    lane-per-row kernel (L 1 is the Motif decode step's call); against selective_scan_pq_ref."""
-    _say(f"pq padded length L={L} R={R}")
+def test_pq_odd_lengths(L, R):
+    """P/Q inference at lengths that are not multiples of 8: the one-step kernel (L 1, the Motif decode
+    step's call), the kernel of four states per lane (4, 5) and the tiled one for any length; against
+    selective_scan_pq_ref."""
+    _say(f"pq odd length L={L} R={R}")
     case = _pq_case(390 + R, batch=2, dim=64, L=L, N=16, R=R, dtype=torch.bfloat16, bkind="4d", G=2)
-    _vs_oracle(case, torch.bfloat16, f"padded L={L}")
+    _vs_oracle(case, torch.bfloat16, f"odd L={L}")
 
 
 def test_pq_rank_zero_is_the_diagonal_scan():

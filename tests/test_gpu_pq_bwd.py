@@ -243,16 +243,17 @@ def test_pq_bwd_c_abi_direct():
 
 
 @pytest.mark.parametrize("L", [12, 1001])
-def test_pq_bwd_padded_lengths(L):
-    """Lengths that are not multiples of 8: the training forward and the backward run on copies
-    padded in front with zero-u steps, which add nothing to any gradient; against the exact ones."""
-    _say(f"pq bwd padded length L={L}")
+def test_pq_bwd_odd_lengths(L):
+    """Lengths that are not multiples of 8: the training forward and the backward take them as they are;
+    against the exact gradients."""
+    _say(f"pq bwd odd length L={L}")
     case = _pq_case(795 + L, batch=2, dim=32, L=L, N=16, R=2, dtype=torch.float32, bkind="4d", G=2)
-    _vs_exact(case, _dout(796, (2, 32, L), torch.float32), torch.float32, f"padded L{L}")
+    _vs_exact(case, _dout(796, (2, 32, L), torch.float32), torch.float32, f"odd L{L}")
 
 
 GENERAL_SHAPES = {
     "dstate20": dict(N=20), "dstate32": dict(N=32), "dstate64": dict(N=64), "dstate32_rank5": dict(N=32, R=5),
+    "dstate64_rank5": dict(N=64, R=5), "dstate33_rank8": dict(N=33, R=8),
     "dstate130": dict(N=130, R=3, dim=8, G=1), "constB": dict(G=1), "constBC": dict(bkind="const"),
     "dim24": dict(dim=24, G=1), "L100": dict(L=100), "shared_pq_dstate32": dict(N=32, per_dim=False),
     # workgroups whose rows span two groups (12 channels per group, 16 rows per workgroup) and two
@@ -266,18 +267,17 @@ GENERAL_SHAPES = {
 
 @pytest.mark.parametrize("what", list(GENERAL_SHAPES))
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-def test_pq_bwd_general_shapes(what, dtype, monkeypatch):
-    """Shapes outside the 16-state kernel run the general P/Q backward (one lane per state, the sums
-    over states as wave butterflies, LDS across waves past 64 states): dstate 20, 32, 64 and 130
-    (the Motif module's "small" and "base" presets use 32 and 64, mamba_simplemotif.py:33-35; the
-    reference's dense kernel takes up to 256), rank 5, a P/Q pair shared by every channel, constant
-    B, constant B and C, 24 and 12 channels (workgroups spanning two groups or two batch rows), L 100
-    with the training padding off; against the exact gradients (dP and dQ included), with z."""
+def test_pq_bwd_general_shapes(what, dtype):
+    """The shapes around the line between scan_bwd_lanes (dstate up to 64, rank up to 4 above 32, variable
+    B and C, channels by 16: dstate 20, 32 and 64, which the Motif module's "small" and "base" presets
+    use, mamba_simplemotif.py:33-35, rank 5 at dstate 32, L 100, a P/Q pair shared by every channel) and
+    the general P/Q backward (one lane per state, the sums over states as wave butterflies, LDS across
+    waves past 64 states: dstate 130, the reference's dense kernel takes up to 256, rank 5 and 8 above
+    dstate 32, constant B, constant B and C, 24 and 12 channels, whose workgroups span two groups or two
+    batch rows); against the exact gradients (dP and dQ included), with z."""
     _say(f"pq bwd general {what} {dtype}")
     kw = dict(batch=2, dim=32, L=64, N=16, R=2, dtype=dtype, bkind="4d", G=2)
     kw.update(GENERAL_SHAPES[what])
-    if what == "L100":
-        monkeypatch.setenv("MM_SCAN_PAD", "0")
     case = _pq_case(790 + len(what), **kw)
     if what == "constB":
         case["B"] = torch.randn(kw["dim"], kw["N"], generator=torch.Generator().manual_seed(791))
@@ -470,11 +470,10 @@ def test_pq_training_step_graph_replay_matches_eager():
 @pytest.mark.parametrize("N,R,L,per_dim", [(16, 2, 15, True), (16, 8, 33, True), (1, 1, 1, True), (17, 4, 16, False),
                                            (32, 8, 31, True), (33, 3, 17, True), (64, 4, 47, False), (63, 2, 32, True)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["fp32", "fp16"])
-def test_pq_bwd_lanes_edges(N, R, L, per_dim, dtype, monkeypatch):
+def test_pq_bwd_lanes_edges(N, R, L, per_dim, dtype):
     """The three lane layouts at the edges of their dstate, rank and tile ranges, on rows of any length
-    and alignment (the training padding off; u, z and dout odd-offset views), two groups."""
+    and alignment (u, z and dout odd-offset views), two groups."""
     _say(f"pq bwd lanes N={N} R={R} L={L} per_dim={per_dim} {dtype}")
-    monkeypatch.setenv("MM_SCAN_PAD", "0")
     case = _pq_case(830 + N + L, batch=2, dim=32, L=L, N=N, R=R, dtype=dtype, bkind="4d", G=2, per_dim=per_dim)
     dout = _dout(831, (2, 32, L), dtype)
     from motif_mamba_amd import selective_scan_fn
