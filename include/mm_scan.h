@@ -137,8 +137,9 @@ typedef struct mm_scan_fwd_params {
      * tile, float32 [ceil(seqlen / 16)][batch][dim][16], states past dstate written as 0 --
      * B * dim * seqlen * 4 bytes, about one float32 copy of u. Passed to mm_scan_bwd as
      * `tile_states`, they spare it the recompute of the whole forward. Written with P/Q and
-     * dstate <= 16, and without P/Q together with chunk_states (the training forward) by the
-     * dstate-16 kernels or, below dstate 16, the P/Q kernels without a coupling
+     * dstate <= 16, and without P/Q together with chunk_states (the training forward) and variable B
+     * and C: at dstate 16 for dim and dim / n_groups multiples of 16, seqlen a multiple of 8 and rows on
+     * 16 bytes, below dstate 16 from 8 steps on
      * (mm_scan_fwd_tile_states_size() is non-zero exactly when this request can write them).
      * NULL: not written. */
     float *tile_states;
@@ -286,8 +287,8 @@ typedef struct mm_state_update_params {
 int mm_scan_fwd(const mm_scan_fwd_params *params, void *stream);
 
 /* Bytes of `workspace` that let mm_scan_fwd use sequence-parallel segments for this request
- * (0: the single-pass kernels are used anyway). Reads only sizes, flags and strides of `params`,
- * and the current device's compute-unit count (the segment count targets three to five waves per SIMD):
+ * (0: the single-pass kernels are used anyway). Reads sizes, flags and strides of `params`, which
+ * pointers are given and how they are aligned, and the current device's compute-unit count (the segment count targets three to five waves per SIMD):
  * query it with the call's device current. Returns 0 for a request mm_scan_fwd would reject. No counterpart in the reference (its forward
  * allocates nothing beyond the outputs, selective_scan.cpp:383-389). */
 int64_t mm_scan_fwd_workspace_size(const mm_scan_fwd_params *params);
@@ -318,8 +319,9 @@ int mm_scan_fwd_noalloc(const mm_scan_fwd_params *params, void *stream);
 int mm_scan_bwd(const mm_scan_bwd_params *params, void *stream);
 
 /* Bytes of `workspace` mm_scan_bwd needs for `params` (0 for a request it would reject or that has
- * nothing to do). Reads sizes and, for dstate 16 with tile_states, the current device's compute-unit
- * count (the size of one round of workgroups). No counterpart in the reference (its backward recomputes each
+ * nothing to do). Reads sizes, flags, strides and which pointers are given, and the current device's
+ * compute-unit count (the size of one round of workgroups; at dstate 32 and 64 it decides between two
+ * kernels): query it with every stride set and the call's device current. No counterpart in the reference (its backward recomputes each
  * 2048-step chunk inside one thread block). */
 int64_t mm_scan_bwd_workspace_size(const mm_scan_bwd_params *params);
 

@@ -571,10 +571,10 @@ int validate_fwd(const mm_scan_fwd_params *p) {
         return fail(MM_ERR_INVALID_ARGUMENT, "mm_scan_fwd: without P/Q, tile_states are written with chunk_states "
                                              "(the training forward)");
     if (p->tile_states && !p->P && !mm::tile_states_ok(*p) && !mm::diag_via_pq_fwd(*p))
-        return fail(MM_ERR_UNSUPPORTED, "mm_scan_fwd: without P/Q, tile_states are written by the dstate-16 kernels "
-                                        "and, below dstate 16, by the P/Q kernels without a coupling (variable "
-                                        "B/C, dim and dim / n_groups multiples of 16, L a multiple of 8, aligned "
-                                        "rows); mm_scan_fwd_tile_states_size tells");
+        return fail(MM_ERR_UNSUPPORTED, "mm_scan_fwd: without P/Q, tile_states are written with variable B/C by the "
+                                        "dstate-16 kernels (dim and dim / n_groups multiples of 16, L a multiple of "
+                                        "8, aligned rows) and, below dstate 16, by the P/Q kernels without a coupling "
+                                        "(8 steps and more); mm_scan_fwd_tile_states_size tells");
     return MM_OK;
 }
 

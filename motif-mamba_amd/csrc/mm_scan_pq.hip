@@ -623,8 +623,9 @@ scan_fwd_pq_tiled(const mm_scan_fwd_params p, const int64_t ratio, const int32_t
 // each, and serve U batch rows with one load of A, P and Q, every row's loads issued before the
 // first is used. The call moves little more than the final states, which leave as 16-byte stores of
 // consecutive lanes (one lane per row wrote each 64-byte state row in 4-byte pieces). No load stands behind
-// a branch or a wait for another, addresses are a uniform base and a 32-bit lane offset, and contiguous
-// rows of A, P and Q come as vectors. Bound by the state writes beyond some 16 batch rows. 64 x 4,096
+// a branch or a wait for another, addresses are a uniform base and a 32-bit lane offset, and a contiguous
+// row of A comes as one vector (of P and Q, too, in the source; the compiler merges their two forms into one
+// set of four-byte loads behind the branch). Bound by the state writes beyond some 16 batch rows. 64 x 4,096
 // channels, dstate 16, rank 2, fp16 (20 MB): 45.4 us per call with one lane per row, 14.1 us here (15.7
 // with a wait per row, per rank and for B and C); 256 rows: 42 us.
 // ------------------------------------------------------------------------------------------------
@@ -723,7 +724,7 @@ scan_fwd_pq_step(const mm_scan_fwd_params p, const int64_t ratio, const int32_t 
             }
         }
     };
-    // One vector per lane and row instead of four loads that each touch every line of the rows.
+    // One vector per lane and row (A) instead of four loads that each touch every line of the rows.
     if (vec & kStepAPQ) {
         const uint32_t n = 4 * uint32_t(n0 < N ? n0 : 0);
         auto four = [&](const float *t, uint32_t off, float *o) {
@@ -929,7 +930,8 @@ scan_fwd_pq_lanes(const mm_scan_fwd_params p, const int64_t ratio) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// dstate past 64: one lane per (batch, channel) row; the row's states in LDS (dstate x 64 floats per
+// dstate past 64 (where no request has tile states) and rows of no step: one lane per (batch, channel)
+// row; the row's states in LDS (dstate x 64 floats per
 // block, lane-minor so every access is conflict-free), P and Q read through the cache.
 // ------------------------------------------------------------------------------------------------
 constexpr int kRowBlock = 64;
@@ -967,11 +969,6 @@ scan_fwd_pq_rowlane(const mm_scan_fwd_params p, const int64_t ratio) {
     const int64_t n_chunks = (L + MM_SCAN_CHUNK - 1) / MM_SCAN_CHUNK;
 
     for (int64_t t = 0; t < L; ++t) {
-        if (p.tile_states && active && t % 16 == 0) {
-            // The state before this 16-step tile, for the backward (states past dstate are 0).
-            float *ck = p.tile_states + ((t / 16) * p.batch * p.dim + b * p.dim + d) * 16;
-            for (int n = 0; n < 16; ++n) ck[n] = n < N ? sH[n * kRowBlock + lane] : 0.f;
-        }
         float dt = to_f32(dp[t]) + bias;
         if (p.delta_softplus) dt = softplus_fast(dt);
         const float uu = to_f32(up[t]);
