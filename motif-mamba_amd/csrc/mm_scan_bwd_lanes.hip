@@ -22,8 +22,9 @@
 // <= 32, 16 x 4 for <= 64), so that the sums over a channel's states that feed the recurrences (Q h
 // and P^T lam) stay inside 16 lanes: one transposed DPP butterfly each (lane_sums, mm_common.h).
 //
-//   * The kernel is bound by VALU issue (two waves per SIMD with a coupling, all the registers its tile
-//     needs), so what a step costs is its instruction count. The states and (S = 2, rank <= 4) decays
+//   * The kernel is bound mostly by VALU issue (82 to 90 % of a SIMD's cycles with a coupling, 77 % at
+//     dstate 64 without one, at two waves per SIMD, all that the registers of its tile allow; the rest
+//     is latency), so what a step costs is its instruction count. The states and (S = 2, rank <= 4) decays
 //     of a 16-step tile stay in registers between the recompute and the reverse walk; the P q term
 //     of dt' is taken as sum_r q_r (P^T lam)_r from the lane's partials and the u B term as
 //     u_t sum_n lam B by the step's owner, so neither costs a multiply per state.
@@ -47,12 +48,12 @@
 //   * The states at every 16-step tile start come from the forward (its tile_states, dstate <= 16)
 //     or from a first pass that recomputes the forward into the caller's workspace.
 //
-// LDS at rank 2: 40 KB (dstate 16), 39 KB (32), 51 KB (64): two waves per SIMD each; 208 registers at
-// dstate 16. About 90 VALU instructions per wave-step of
-// 8 channels x 16 states.
+// LDS at rank 2: 40 KB (dstate 16), 39 KB (32), 51 KB (64): two waves per SIMD each; 188 registers at
+// dstate 16. 85 VALU instructions per wave-step of 8 channels x 16 states, 114 of 4 x 32. Rank 4 above
+// dstate 32 spills 32 to 37 registers, the other instances at most one.
 //
 // Measured (rank 2, per-channel P/Q), training step of forward and backward: batch 4, 4,096 channels,
-// L 2,048, dstate 16, fp16: 1.55 -> 1.27 ms (backward 1.19 -> 0.93) against a kernel with the tile's
+// L 2,048, dstate 16, fp16: 1.55 -> 1.26 ms (backward 1.19 -> 0.92) against a kernel with the tile's
 // states in LDS, DPP butterflies for the du / ddelta sums and 124 VALU per wave-step; batch 8, 1,024
 // channels, L 1,024, dstate 32, bf16: 4.39 -> 0.78 ms against one lane per state.
 //
