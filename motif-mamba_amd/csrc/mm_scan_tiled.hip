@@ -1910,8 +1910,8 @@ static int64_t min_ragged(const mm_scan_fwd_params &p) {
 // Requests of any length and row alignment that the ragged k2s takes: inference (no chunk or tile
 // states, one output), from min_ragged steps on.
 static bool ragged_ok(const mm_scan_fwd_params &p) {
-    if (!has_rows(p) || p.dstate != 16 || !p.is_variable_B || !p.is_variable_C || p.chunk_states || p.tile_states || (p.z && p.out))
-        return false;
+    if (!has_rows(p) || (p.z && p.out) || p.chunk_states || p.tile_states) return false;
+    if (p.dstate != 16 || !p.is_variable_B || !p.is_variable_C) return false;
     if (p.dim % tiled::kCh != 0 || (p.dim / p.n_groups) % tiled::kCh != 0) return false;
     // Rows start on whole elements.
     const uintptr_t eb = p.itype == MM_FLOAT32 ? 4 : 2;
@@ -1959,11 +1959,11 @@ int64_t device_simds() {
 }
 
 // Sequence segments for shapes whose (batch, 16-channel) groups give fewer than one wave per SIMD
-// (two waves per group). Up to 1,504 steps (47 tile pairs) rows are cut in two at most, from 1,024 on:
+// (two waves per group). Rows of 32 to 47 tile pairs (993 to 1,504 steps) are cut in two, shorter ones not:
 // two segments keep the bits of the whole row (the second starts from the first's end state as it is), and
 // so inference those of the training forward, which is not cut; the carry of three and more reassociates
 // sums. (1 x 5,120 channels, L 1,024, bf16: 68 us in two, 70 whole. More segments would be faster: 512, L
-// 1,024: 19 us in 16, 46 whole or in two; 2,560, L 1,280: 37 in 13, 70 in two.)
+// 1,024: 19 us in 16, 46 whole or in two; 2,560, L 1,280: 37 in 8, 70 in two.)
 // Past that, two plans: as many segments of at least 64 steps as give three waves per SIMD, or of at least
 // 512 steps as give five, whichever needs fewer rounds of waves per step of a segment. bf16,
 // against at most five waves per SIMD of at least 512 steps: 512 channels, L 2,048: 47 -> 22 us; 1,536,

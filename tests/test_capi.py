@@ -184,8 +184,8 @@ def test_workspace_size_query():
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(params(4, 5120, 4096))) == 0   # config 2: one pass
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(params(1, 64, 256))) == 0      # too short to split
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(params(1, 64, 8192, N=32))) == 0  # not dstate 16
-    # Two segments at most up to 1,504 steps (those keep the whole row's bits), none below 1,024.
-    for L, n_seg in ((992, 0), (1024, 2), (1280, 2), (1504, 2)):
+    # Two segments from 32 to 47 tile pairs of 32 steps (two keep the whole row's bits), none below.
+    for L, n_seg in ((992, 0), (1000, 2), (1024, 2), (1280, 2), (1504, 2)):
         assert lib.mm_scan_fwd_workspace_size(ctypes.byref(params(1, 64, L))) == 64 * n_seg * 18 * 4, L
     assert lib.mm_scan_fwd_workspace_size(ctypes.byref(params(1, 64, 1536))) > 64 * 2 * 18 * 4
     bad = params(1, 64, 8192)
